@@ -17,8 +17,9 @@ namespace {
 constexpr int kNumConfigs = 17;
 constexpr int kSmallMConfigs = 3;  // ids 0..2: small-M kernel, M <= kSmallMMax
 constexpr int kSmallMMax = 64;
-constexpr int kTiledConfigs = 4;   // ids 3..6: MFMA-tiled kernel, any M
-constexpr int kStreamFirst = kSmallMConfigs + kTiledConfigs;  // ids 7..9: streaming kernel, M <= 16
+constexpr int kWideFirst = kSmallMConfigs;  // ids 3..6: wide-tile kernel, any M
+constexpr int kWideConfigs = 4;
+constexpr int kStreamFirst = kWideFirst + kWideConfigs;  // ids 7..9: streaming kernel, M <= 16
 constexpr int kStreamMax = 16;
 constexpr int kStreamConfigs = 3;
 constexpr int kPrefillFirst = kStreamFirst + kStreamConfigs;  // ids 10..13: prefill kernel, any M
@@ -192,13 +193,11 @@ void run_gemm(int W, int A, int config, int mode, const LinearArgs& g, hipStream
     launch_smallm(W, A, kSmallMWaves[config], mode, g, st);
     return;
   }
-  for (int p = 0; p < g.nprob; ++p) {
-    LinearArgs one = g;
-    one.prob[0] = g.prob[p];
-    one.prob[0].tile0 = 0;
-    one.nprob = 1;
-    launch_tiled(W, A, config - kSmallMConfigs, mode == kModeDots, one, st);
-  }
+  const int shape = config - kWideFirst;
+  if (mode == kModeDots) launch_prefill(W, A, shape, true, g, st);  // (single problem)
+  else if (W == 8) launch_wide_w8(A, shape, g, st);
+  else if (W == 4) launch_wide_w4(A, shape, g, st);
+  else launch_wide_w2(A, shape, g, st);
 }
 
 LinearArgs base_args(int64_t M, int64_t K, int bias_dt, int out_dt) {
@@ -384,14 +383,116 @@ int packed_default(int64_t M, int64_t N, int64_t K, int W, int A) {
   // workgroups for small problems), 128x64 tiles for W <= 4 from four tiles
   // per CU (each unpacked weight slot feeds twice the tokens; 2-7% faster at
   // N=16384 M=256 and N=4096 M=1024; W8's 128x64 tiles hold too many
-  // registers for two waves per SIMD), and the LDS-staged tiled kernel for
-  // the largest problems, whose 4-wave 64x64 tiles share weight fragments in
-  // LDS.
+  // registers for two waves per SIMD), and the wide-tile kernel for the
+  // largest problems. Calls under ACTUNE_CONFIG_AUTO above 16 tokens go on to
+  // run_planned.
   const int64_t t64 = ((N + 63) / 64) * ((M + 63) / 64);
   if (t64 < 512) return kPrefillFirst + 3;
   if (t64 < 1024) return kPrefillFirst + 2;
   if (t64 < 2048) return W <= 4 ? kPrefillFirst + 0 : kPrefillFirst + 2;
-  return kSmallMConfigs;
+  return kWideFirst;
+}
+
+// Kernel of a call on codes above 16 tokens under ACTUNE_CONFIG_AUTO: the
+// least estimated time (us) among the decode kernel (up to 64 tokens), the
+// wide-tile kernel over all problems in one launch, and the prefill kernel
+// problem by problem. A launch costs about 6.5 us beyond its walk over K
+// (prologue and epilogue included), the walk K / 4096 times what its
+// TileCost says for the launch's tile count: whole rounds over the 256 CUs where a
+// workgroup fills a CU, measured at one and two workgroups per CU and then
+// proportional to the tiles where several fit.
+// Measured on MI355X (us, K = 4096, hipGraph, rotating weights; W8A8 at N =
+// 4096 / 11008 / 22016, M = 20 .. 2000, and W4A8, W4A4 likewise): W8 128x128
+// tiles 33 per round of 256, 64x128 22, 64x64 18 / 26 up to one / two per CU,
+// prefill 64x32 15.5 up to one per CU; W4 128x64 25 / 38, 64x64 18 / 25,
+// 128x32 16.5 per round, prefill 64x32 11.8, 64x64 17.5 / 24, 128x64 24.5 /
+// 37.5. The decode kernel takes 11.3 (W8: 21) per 1024 blocks of 16 rows x 16
+// tokens, the small-M kernel that stands in for a long K 20 (21). Before
+// this rule 17-64 tokens always took the decode or small-M kernel, and
+// siblings the configuration of their total N: W4A8 11008x4096 at M = 40
+// 27.5 -> 16.2, 4096x11008 at M = 64 44.2 -> 21.6, W8A8 22016x4096 at M = 64
+// 83.8 -> 28.4, 4096x11008 at M = 1024 134.8 -> 87.9.
+struct TileCost {
+  int bn, bm;           // tile: rows x tokens
+  float one, two, per;  // up to 256 and 512 tiles; per tile above (0: `one` per round of 256)
+};
+constexpr TileCost kWideCost[2][3] = {{{128, 64, 25.f, 38.f, 0.0725f}, {64, 64, 18.f, 25.f, 0.0425f}, {128, 32, 16.5f, 0, 0}},
+                                      {{128, 128, 33.f, 0, 0}, {64, 64, 18.f, 26.f, 0.0487f}, {64, 128, 22.f, 0, 0}}};
+// prefill configs 10, 12, 13
+constexpr TileCost kPrefillCost[2][3] = {{{128, 64, 24.5f, 37.5f, 0.0785f}, {64, 64, 17.5f, 24.f, 0.041f}, {64, 32, 11.8f, 16.f, 0.036f}},
+                                         {{128, 64, 28.f, 54.f, 0.12f}, {64, 64, 18.5f, 28.f, 0.055f}, {64, 32, 15.5f, 25.f, 0.054f}}};
+constexpr int kPrefillCostConfig[3] = {kPrefillFirst, kPrefillFirst + 2, kPrefillFirst + 3};
+constexpr float kLaunchCost = 6.5f;
+
+int64_t tiles_of(const TileCost& c, int64_t M, int64_t N) { return ((N + c.bn - 1) / c.bn) * ((M + c.bm - 1) / c.bm); }
+
+float launch_cost(const TileCost& c, int64_t tiles, int64_t K) {
+  float t;
+  if (c.per == 0.f) t = c.one * (float)((tiles + 255) / 256);
+  else t = tiles <= 256 ? c.one : tiles <= 512 ? c.two : std::max(c.two, c.per * (float)tiles);
+  return kLaunchCost + (float)K / 4096.f * (t - kLaunchCost);
+}
+
+// The prefill config of one problem, and its estimated time.
+int prefill_choice(int64_t M, int64_t N, int64_t K, int W, float* us) {
+  int best = 0;
+  for (int i = 0; i < 3; ++i) {
+    const TileCost& c = kPrefillCost[W == 8][i];
+    const float t = launch_cost(c, tiles_of(c, M, N), K);
+    if (i == 0 || t < *us) { *us = t; best = i; }
+  }
+  return kPrefillCostConfig[best];
+}
+
+// Runs the problems of g (one width, M > 16) on codes with the kernel of the
+// least estimated time.
+void run_planned(int W, int A, const LinearArgs& g, hipStream_t st) {
+  const int64_t M = g.M, K = g.K;
+  int64_t n_total = 0;
+  for (int q = 0; q < g.nprob; ++q) n_total += g.prob[q].N;
+  const int single = packed_default(M, n_total, K, W, A);
+  if (M > kDecodeAutoMax && single >= kDecodeFirst) {  // narrow problems keep the decode kernel
+    run_gemm(W, A, single, kModePacked, g, st);
+    return;
+  }
+  float best = 0.f, us = 0.f;
+  int config = -1;  // one launch over every problem; -1: prefill, problem by problem
+  for (int q = 0; q < g.nprob; ++q) {
+    prefill_choice(M, g.prob[q].N, K, W, &us);
+    best += us;
+  }
+  for (int i = 0; i < 3; ++i) {
+    const TileCost& c = kWideCost[W == 8][i];
+    int64_t tiles = 0;
+    for (int q = 0; q < g.nprob; ++q) tiles += tiles_of(c, M, g.prob[q].N);
+    us = launch_cost(c, tiles, K);
+    if (us <= best) { best = us; config = kWideFirst + i; }
+  }
+  if (M <= kDecodeAutoMax) {
+    const bool fits = single >= kDecodeFirst;
+    const float blocks = (float)((n_total + 15) / 16 * ((M + 15) / 16));
+    us = (float)K / 4096.f * blocks / 1024.f * (W == 8 ? 21.f : fits ? 11.3f : 20.f);
+    if (us <= best) config = single;
+  }
+  if (config >= 0) {
+    run_gemm(W, A, config, kModePacked, g, st);
+    return;
+  }
+  for (int q = 0; q < g.nprob; ++q) {
+    LinearArgs one = g;
+    one.prob[0] = g.prob[q];
+    one.prob[0].tile0 = 0;
+    one.nprob = 1;
+    one.tiles = (g.prob[q].N + 15) / 16;
+    run_gemm(W, A, prefill_choice(M, g.prob[q].N, K, W, &us), kModePacked, one, st);
+  }
+}
+
+// Runs the problems of g on codes: `config`, or under ACTUNE_CONFIG_AUTO above
+// 16 tokens the planned kernel.
+void run_codes(int W, int A, int config, bool auto_config, const LinearArgs& g, hipStream_t st) {
+  if (auto_config && g.M > kStreamMax) run_planned(W, A, g, st);
+  else run_gemm(W, A, config, kModePacked, g, st);
 }
 }  // namespace
 
@@ -427,6 +528,7 @@ int actune_grouped_linear(const uint8_t* a, const float* a_scales, const uint8_t
                           int out_dtype, int64_t M, int64_t N, int64_t K, int W, int A, int config,
                           void* stream) {
   g_err[0] = 0;
+  const bool auto_config = config == ACTUNE_CONFIG_AUTO;
   config = resolve(config, M, N, K, W, A, false);
   int rc = check_shape(M, K, W, A, out_dtype, bias_dtype, config);
   if (!rc) rc = check_target(w, w_scale, out, N, M, K, W);
@@ -437,7 +539,7 @@ int actune_grouped_linear(const uint8_t* a, const float* a_scales, const uint8_t
   g.a = a;
   g.as = a_scales;
   add_problem(g, w, w_scale, bias, out, N, W);
-  run_gemm(W, A, config, kModePacked, g, (hipStream_t)stream);
+  run_codes(W, A, config, auto_config, g, (hipStream_t)stream);
   return check_launch();
 }
 
@@ -487,7 +589,7 @@ int forward_mixed(LinearArgs& g, int config, bool auto_config, int64_t n_total, 
         n_w += g.prob[r].N;
         done[r] = true;
       }
-    run_gemm(w, A, auto_config ? packed_default(g.M, n_w, g.K, w, A) : config, kModePacked, one, st);
+    run_codes(w, A, auto_config ? packed_default(g.M, n_w, g.K, w, A) : config, auto_config, one, st);
   }
   return check_launch();
 }
@@ -539,7 +641,7 @@ int actune_grouped_forward_multi(const void* x, int x_dtype, const void* input_s
     launch_quantize(x, x_dtype, input_scale, M, K, A, a_buf, scale_buf, st);
     g.a = a_buf;
     g.as = scale_buf;
-    run_gemm(W, A, config, kModePacked, g, st);
+    run_codes(W, A, config, auto_config, g, st);
   }
   return check_launch();
 }

@@ -1,0 +1,8 @@
+// The wide-tile kernel (gemm_wide.hpp) for W8 weights.
+#include "gemm_wide.hpp"
+
+namespace actune {
+
+void launch_wide_w8(int A, int shape, const LinearArgs& g, hipStream_t st) { launch_wide_width<8>(A, shape, g, st); }
+
+}  // namespace actune

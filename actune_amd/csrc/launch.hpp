@@ -99,7 +99,10 @@ void launch_quantize(const void* x, int dt, const void* sc, long M, long K, int 
 void launch_quantize_gated(const void* gate, const void* up, int dt, int act, const void* sc, long M, long K, int A,
                            uint8_t* packed, float* scales, hipStream_t stream);
 void launch_smallm(int W, int A, int nw, int mode, const LinearArgs& g, hipStream_t st);
-void launch_tiled(int W, int A, int shape, bool dots, const LinearArgs& g, hipStream_t st);
+// the wide-tile kernel on packed codes, every problem of g (one width) in one launch
+void launch_wide_w2(int A, int shape, const LinearArgs& g, hipStream_t st);
+void launch_wide_w4(int A, int shape, const LinearArgs& g, hipStream_t st);
+void launch_wide_w8(int A, int shape, const LinearArgs& g, hipStream_t st);
 void launch_stream(int W, int A, int nw, int mode, const LinearArgs& g, hipStream_t st);
 void launch_prefill(int W, int A, int shape, bool dots, const LinearArgs& g, hipStream_t st);
 // packed: the activations are codes + scales from the quantizer launch

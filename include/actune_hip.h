@@ -160,7 +160,9 @@ int actune_grouped_dots_i32(const uint8_t* a, const uint8_t* w, int64_t M, int64
  * Kernel configurations, the counterpart of the 13 tile geometries of
  * actune/kernels/grouped_big_m.cu:115-130 selected by tuning.py:16-45.
  *   0, 1, 2  small-M split-K kernel with 4, 8, 16 waves (M <= 64)
- *   3 .. 6   MFMA-tiled kernel shapes (any M)
+ *   3 .. 6   wide-tile kernel (any M): 128x64 (W8 128x128), 64x64, 128x32 with
+ *            K split in two (W8 64x128), 64x32 with K split in four (W8 two);
+ *            the dots mode runs the prefill kernel
  *   7, 8, 9  persistent streaming kernel with 4, 8, 16 waves (M <= 16)
  *   10 .. 13 prefill kernel (weights streamed per wave, activations staged
  *            per workgroup) with tiles 128x64, 128x32, 64x64, 64x32 (any M)
@@ -176,7 +178,8 @@ int actune_grouped_dots_i32(const uint8_t* a, const uint8_t* w, int64_t M, int64
  *   actune_grouped_forward(_multi). actune_grouped_linear and
  *   actune_grouped_dots_i32 (packed activations) resolve AUTO to the same
  *   kernels without the in-launch quantization (a decode config where the
- *   decode kernel fits the codes). For a width or dimension that no call
+ *   decode kernel fits the codes). Above 16 tokens an AUTO call on codes runs
+ *   the kernel of the least estimated time instead (bit-identical). For a width or dimension that no call
  *   takes it returns ACTUNE_CONFIG_AUTO (-1); a call with such arguments
  *   returns ACTUNE_ERR_INVALID naming them, whatever its config.
  */
