@@ -65,6 +65,8 @@ def lib():
                                                  _P, _I64, _P]
         so.actune_tokenwise_linear_multi.argtypes = [_P, _I, _P, _I, _P, _I, ctypes.POINTER(_TwTarget), _I, _I, _I,
                                                      _I64, _I64, _I64, _I, _P, _I64, _P]
+        so.actune_weight_candidates.argtypes = [_P, _I, _P, _I, _I64, _I64, _I, _I, _P, _P, _P]
+        so.actune_candidate_select.argtypes = [_P, _P, _P, _I, _I64, _I64, _P, _P, _P, _P]
         so.actune_forward_fuses_quantizer.argtypes = [_I64, _I64, _I64, _I, _I, _I, _I]
         so.actune_config_valid.argtypes = [_I, _I64]
         so.actune_default_config.argtypes = [_I64, _I64, _I64, _I, _I]
@@ -265,6 +267,40 @@ def quantize_gated(gate: torch.Tensor, up: torch.Tensor, act: int, a: int, input
     _check(lib().actune_quantize_gated(_ptr(gate), _ptr(up), _dtype_code(gate), act, _ptr(input_scale), m, k, a,
                                        _ptr(packed), _ptr(scales), _stream(gate.device)))
     return packed, scales
+
+
+def weight_candidates(weight, ratios, w, a):
+    """Packed codes u8 [R * N, K*w/8] and scales f32 [R * N] of a contiguous
+    [N, K] weight under each clip ratio of the f32 device tensor `ratios`
+    (actune_weight_candidates)."""
+    _require_cuda(weight, ratios)
+    _check_widths(w, a)
+    _check_flat(weight)
+    if ratios.dtype != torch.float32 or ratios.dim() != 1 or not ratios.is_contiguous():
+        raise RuntimeError("ratios must be a contiguous float32 vector")
+    weight = _aligned16(weight)
+    n, k = weight.shape
+    rows = ratios.numel() * n
+    packed = torch.empty((rows, k * w // 8), device=weight.device, dtype=torch.uint8)
+    scales = torch.empty(rows, device=weight.device, dtype=torch.float32)
+    _check(lib().actune_weight_candidates(_ptr(weight), _dtype_code(weight), _ptr(ratios), ratios.numel(), n, k, w, a,
+                                          _ptr(packed), _ptr(scales), _stream(weight.device)))
+    return packed, scales
+
+
+def candidate_select(y, ref, ratios, best, chosen):
+    """Losses [R, N] of the candidates' fp32 outputs y [M, R * N] against ref
+    [M, N]; best / chosen [N] keep each row's lowest loss and its ratio
+    (actune_candidate_select)."""
+    _require_cuda(y, ref, ratios, best, chosen)
+    (m, n), r = ref.shape, ratios.numel()
+    for t, name, shape in ((y, "y", (m, r * n)), (ref, "ref", (m, n)), (ratios, "ratios", (r,)),
+                           (best, "best", (n,)), (chosen, "chosen", (n,))):
+        _check_buffer(t, name, shape, torch.float32, ref.device)
+    loss = torch.empty((r, n), device=ref.device, dtype=torch.float32)
+    _check(lib().actune_candidate_select(_ptr(y), _ptr(ref), _ptr(ratios), r, m, n, _ptr(loss), _ptr(best),
+                                         _ptr(chosen), _stream(ref.device)))
+    return loss
 
 
 def _check_linear_operands(a, as_, w, ws, bias, m, k, n, W, A):

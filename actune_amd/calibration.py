@@ -16,9 +16,11 @@ Same contract as actune/calibration.py:7-16 and :42-93:
   operands with a float GEMM (F.linear of dequantized activations and
   weights); both are fp32 evaluations of the same exact sums, so scores
   differ only in the last bits and the selected scale and clips agree except
-  on exact near-ties.
-* Weight codebooks are evaluated with torch on the layer's device, as the
-  reference does (quantizers.py:23-94): on a GPU the divisions by the
+  on exact near-ties. All clip ratios of a pair are evaluated together: their
+  packed weights stand one below the other, so one launch forms the codes, one
+  GEMM the outputs and one kernel the losses.
+* Weight codebooks are torch's on the layer's device, as the reference
+  evaluates them (quantizers.py:23-94): on a GPU the divisions by the
   constants 7 and 127 are reciprocal multiplies there as well.
 
 Calibration runs on the GPU only: CPU tensors raise ValueError (the
@@ -31,7 +33,6 @@ from __future__ import annotations
 import torch
 
 from . import _native
-from .kernels.grouped import pack_rows
 
 _CLIP_GRID = (1., .975, .95, .925, .9, .875, .85, .8, .75)
 
@@ -68,39 +69,50 @@ def activation_reference(value, bits, group_size=64):
     return deq.reshape(shape)
 
 
-def _clip(weight_rows, ratio):
-    return weight_rows if ratio is None else weight_rows * ratio
+def _ratios(values, device):
+    return torch.tensor([1.0 if v is None else float(v) for v in values], dtype=torch.float32, device=device)
 
 
 def _codes_on_device(weight, w, a, ratio):
-    """weight_codes (quantizers.py:23-94) evaluated by torch on the weight's
-    device; ratio is a float in (0, 1] or None."""
-    value = weight.detach().float()
-    amax = value.abs().amax(dim=1).clamp_min(1e-8)
-    if w == 8 and a != 4:
-        scale = amax / 127.0
-        return (value / scale[:, None]).round().clamp(-128, 127).to(torch.int8), scale
-    amax = _clip(amax, ratio)
-    if w == 2:
-        return (value / amax[:, None]).round().clamp(-2, 1).to(torch.int8), amax
-    scale4 = amax / 7.0
-    q4 = (value / scale4[:, None]).round().clamp(-8, 7).to(torch.int8)
-    if w == 4:
-        return q4, scale4
-    residual = (16.0 * (value / scale4[:, None] - q4.float())).round().clamp(-8, 7).to(torch.int16)
-    q4i = q4.to(torch.int16)
-    residual = torch.minimum(torch.maximum(residual, (-128 - 16 * q4i).clamp_min(-8)), (127 - 16 * q4i).clamp_max(7))
-    return (16 * q4i + residual).to(torch.int8), scale4 / 16.0
+    """weight_codes (quantizers.py:23-94) with torch's GPU division, by the
+    candidates kernel; ratio is a float in (0, 1] or None."""
+    packed, scale = _native.weight_candidates(weight.detach().contiguous(), _ratios((ratio,), weight.device), w, a)
+    return _unpack_codes(packed, w, weight.shape[1]), scale
+
+
+def _outputs(a_codes, weight, w, a, ratios):
+    """fp32 outputs [M, R * N] of the packed GEMM for the codes of x against
+    the weight candidates of every ratio, one below the other."""
+    a_packed, a_scales = a_codes
+    packed, scale = _native.weight_candidates(weight, ratios, w, a)
+    return _native.grouped_linear(a_packed, a_scales, packed, scale, None, (a_packed.shape[0], weight.shape[1]), w, a,
+                                  out_dtype=torch.float32)
 
 
 def _candidate(x_scaled, weight, w, a, ratio):
     """fp32 output of the packed GEMM for x_scaled (already divided by the
     channel scale, in the layer dtype) against weight codes (w, a, ratio)."""
-    codes, scale = _codes_on_device(weight, w, a, ratio)
-    packed = pack_rows(codes, w)
-    a_packed, a_scales = _native.quantize_groups(x_scaled, a)
-    return _native.grouped_linear(a_packed, a_scales, packed, scale.contiguous(), None,
-                                  tuple(x_scaled.shape), w, a, out_dtype=torch.float32)
+    return _outputs(_native.quantize_groups(x_scaled, a), weight.detach().contiguous(), w, a,
+                    _ratios((ratio,), weight.device))
+
+
+# fp32 outputs and packed weights of the candidates evaluated at a time
+_CANDIDATE_BYTES = 512 << 20
+
+
+def _best_candidates(a_codes, weight, w, a, grid, reference):
+    """(loss, ratio) per row of the first candidate of the lowest loss over
+    the ratios of the f32 device tensor `grid`, and the last losses."""
+    m, n = reference.shape
+    best = torch.full((n,), float("inf"), device=reference.device)
+    chosen, losses = torch.ones_like(best), None
+    if w == 8 and a != 4:
+        grid = grid[:1]  # plain W8 takes no clip: every candidate is the first
+    step = max(1, _CANDIDATE_BYTES // (n * max(4 * m, weight.shape[1] * w // 8)))
+    for i in range(0, len(grid), step):
+        ratios = grid[i:i + step]
+        losses = _native.candidate_select(_outputs(a_codes, weight, w, a, ratios), reference, ratios, best, chosen)
+    return best, chosen, losses
 
 
 @torch.no_grad()
@@ -125,31 +137,33 @@ def calibrate_linear(linear, inputs, row_weights=None, *, budget="w4a4", group_s
     reference = torch.nn.functional.linear(x.float(), linear.weight.float())
     base_a = 4 if budget == "w4a4" else 8
     moment = x.float().abs().mean(0).clamp_min(1e-4)
-    best = None
+    x, unclipped = x.contiguous(), torch.ones(1, device=x.device)
+    candidates, scores = [], []
     for alpha in (0., .25, .5, .75, 1.):
         scale = moment.pow(alpha)
         scale = (scale / (scale.max() * scale.min()).sqrt()).clamp(1 / 16, 16).to(x.dtype)
-        weight = (linear.weight * scale[None, :]).to(x.dtype)
-        y = _candidate((x / scale).contiguous(), weight, 4, base_a, None)
-        score = float(((y - reference).square().mean(0) * gains).sum())
-        if best is None or score < best[0]:
-            best = score, scale
-    scale = best[1]
-    weight = (linear.weight * scale[None, :]).to(x.dtype)
-    x_scaled = (x / scale).contiguous()
-    errors, clips = {}, {}
+        weight = (linear.weight * scale[None, :]).to(x.dtype).contiguous()
+        _, _, losses = _best_candidates(_native.quantize_groups(x, base_a, scale), weight, 4, base_a, unclipped,
+                                        reference)
+        candidates.append((scale, weight))
+        scores.append((losses[0] * gains).sum())
+    scores = torch.stack(scores).tolist()
+    chosen = 0
+    for i, score in enumerate(scores):
+        if score < scores[chosen]:
+            chosen = i
+    scale, weight = candidates[chosen]
+    widths = (8,) if budget == "w4a8" else (2, 4, 8)
+    a_codes = {a: _native.quantize_groups(x, a, scale) for a in widths}
+    grid = tuple(clip_grid)
+    if not all(0 < ratio <= 1 for ratio in grid):
+        raise ValueError("Clip ratios must lie in (0, 1]")
+    grid = _ratios(grid, x.device)
+    totals, clips = {}, {}
     for w in (2, 4, 8):
-        for a in ((8,) if budget == "w4a8" else (2, 4, 8)):
-            row_error = torch.full((linear.out_features,), float("inf"), device=x.device)
-            selected = torch.ones_like(row_error)
-            for ratio in clip_grid:
-                if not 0 < ratio <= 1:
-                    raise ValueError("Clip ratios must lie in (0, 1]")
-                output = _candidate(x_scaled, weight, w, a, ratio)
-                loss = (output - reference).square().mean(0)
-                improve = loss < row_error
-                selected[improve], row_error[improve] = ratio, loss[improve]
+        for a in widths:
             mode = f"w{w}a{a}"
-            errors[mode] = float((row_error * gains).sum())
-            clips[mode] = selected
+            row_error, clips[mode], _ = _best_candidates(a_codes[a], weight, w, a, grid, reference)
+            totals[mode] = (row_error * gains).sum()
+    errors = dict(zip(totals, torch.stack(list(totals.values())).tolist()))
     return dict(channel_scale=scale, clips=clips, errors=errors, group_size=group_size)

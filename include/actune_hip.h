@@ -319,6 +319,26 @@ int actune_tokenwise_linear_multi(const void* a, int a_layout, const void* x, in
  */
 int actune_layout_selftest(void);
 
+/*
+ * Calibration: the packed weight candidates of one layer and the choice among
+ * their outputs (actune/kernels/quantizers.py:23-94, calibration.py:74-88).
+ *
+ * actune_weight_candidates: codes and scales of w [N, K] (bf16 / f16 / f32,
+ * 16-byte aligned) for width W used with activation width A under each of the
+ * R clip ratios (device memory), the divisions by 7 and 127 as torch computes
+ * them on a GPU. Candidate r is rows r N .. r N + N - 1 of packed
+ * [R N, K W / 8] and scales [R N]. Plain W8 (A != 4) ignores the ratios.
+ *
+ * actune_candidate_select: y [M, R N] are the fp32 outputs of R candidates,
+ * ref [M, N] the reference. loss [R N] receives each row's mean squared
+ * difference (scratch); where a candidate's loss is strictly below best[n], in
+ * order of r, best[n] and chosen[n] become its loss and ratio.
+ */
+int actune_weight_candidates(const void* w, int w_dtype, const float* ratios, int R, int64_t N, int64_t K, int W, int A,
+                             uint8_t* packed, float* scales, void* stream);
+int actune_candidate_select(const float* y, const float* ref, const float* ratios, int R, int64_t M, int64_t N,
+                            float* loss, float* best, float* chosen, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
