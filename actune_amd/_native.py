@@ -11,6 +11,7 @@ messages (actune/kernels/grouped_native.cu:92-105, grouped.py:118-119, 128).
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 from pathlib import Path
 
 import torch
@@ -72,6 +73,30 @@ def lib():
         so.actune_default_config.argtypes = [_I64, _I64, _I64, _I, _I]
         _LIB = so
     return _LIB
+
+
+FAST_PATH = LIB_PATH.parent / "_actune_fast.so"
+_FAST = None
+# the functions the native call path runs, in the order its init() takes them
+_FAST_API = ("actune_quantize_groups", "actune_quantize_gated", "actune_grouped_linear", "actune_grouped_forward_multi",
+             "actune_tokenwise_quantize", "actune_tokenwise_workspace_bytes", "actune_tokenwise_linear",
+             "actune_tokenwise_linear_x", "actune_tokenwise_linear_multi", "actune_last_error")
+
+
+def fast():
+    """The native call path (csrc/binding.cpp) over the loaded library: its
+    functions take the plain case of the calls below, or return None."""
+    global _FAST
+    if _FAST is None:
+        so = lib()
+        if not FAST_PATH.exists():
+            raise ImportError(f"{FAST_PATH} is missing: build it with `python -m actune_amd.build`")
+        spec = importlib.util.spec_from_file_location("_actune_fast", FAST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.init([ctypes.cast(getattr(so, name), _P).value for name in _FAST_API])
+        _FAST = module
+    return _FAST
 
 
 def _check(rc: int) -> None:
@@ -232,6 +257,10 @@ def _act_buffers(packed, scales, m, k, a, device):
 def quantize_groups(x: torch.Tensor, a: int, input_scale: torch.Tensor | None = None,
                     packed: torch.Tensor | None = None, scales: torch.Tensor | None = None):
     """Group-64 quantize a contiguous [M, K] tensor; returns (packed, scales)."""
+    if packed is None and scales is None:
+        done = fast().quantize_groups(x, a, input_scale)
+        if done is not None:
+            return done
     _require_cuda(x, input_scale, packed, scales)
     _check_widths(8, a)
     _check_flat(x)
@@ -253,6 +282,10 @@ def quantize_gated(gate: torch.Tensor, up: torch.Tensor, act: int, a: int, input
     formed in the inputs' dtype as torch forms it) through
     actune_quantize_gated: equal to quantize_groups on a tensor holding p.
     gate, up: contiguous [M, K] of one dtype. Returns (packed, scales)."""
+    if packed is None and scales is None and act in (ACT_SILU, ACT_GELU_TANH):
+        done = fast().quantize_gated(gate, up, act, a, input_scale)
+        if done is not None:
+            return done
     _require_cuda(gate, up, input_scale, packed, scales)
     _check_widths(8, a)
     _check_flat(gate)
@@ -329,6 +362,15 @@ def grouped_linear(a, as_, w, ws, bias, source_or_shape, W, A, config=CONFIG_AUT
     packed activations + scales x packed weights -> [M, N] in source.dtype.
     ``source_or_shape`` is the [M, K] source tensor (its dtype and shape
     define the output), as in the reference op signature."""
+    if out is None:
+        if isinstance(source_or_shape, torch.Tensor):
+            shape, dtype = source_or_shape.shape, source_or_shape.dtype
+        else:
+            shape, dtype = source_or_shape, out_dtype or torch.bfloat16
+        if len(shape) == 2:
+            done = fast().grouped_linear(a, as_, w, ws, bias, *shape, DTYPE_CODES.get(dtype, -1), W, A, config)
+            if done is not None:
+                return done
     _require_cuda(a, as_, w, ws, bias)
     if isinstance(source_or_shape, torch.Tensor):
         m, k = source_or_shape.shape
@@ -357,6 +399,10 @@ def grouped_forward(flat, w, ws, bias, W, A, input_scale=None, config=CONFIG_AUT
     """Quantize + GEMM for a contiguous [M, K] input (GroupedLinear.forward's
     device work, grouped.py:127-143); returns [M, N] in flat.dtype.
     packed [M, K*A/8] / scales [M, K/64] / out may be preallocated."""
+    if out is None and packed is None and scales is None:
+        done = fast().grouped_forward(flat, w, ws, bias, W, A, input_scale, config)
+        if done is not None:
+            return done
     _require_cuda(flat, w, ws, bias, input_scale, out, packed, scales)
     _check_widths(W, A)
     _check_flat(flat)
@@ -383,6 +429,10 @@ def grouped_forward_multi(flat, targets, W, A, input_scale=None, config=CONFIG_A
     W_t differs from W (the call then runs the widths in one decode launch
     where the kernel takes them, else one launch per width on one
     quantization). Returns the list of outputs."""
+    if packed is None and scales is None:
+        done = fast().grouped_forward_multi(flat, targets, W, A, input_scale, config)
+        if done is not None:
+            return done
     if not 1 <= len(targets) <= MAX_TARGETS:
         raise ValueError("between 1 and 4 targets required")
     _require_cuda(flat, input_scale, packed, scales, *[t for tgt in targets for t in tgt[:4]])
@@ -448,6 +498,10 @@ TW_EPI_A8, TW_EPI_A4 = 0, 1
 def tokenwise_quantize(x, bits, codes=None, scales=None):
     """Per-row dynamic A8 (int8 [M, K]) or A4 (packed u8 [M, K/2]) codes and
     f32 [M] scales of a contiguous [M, K] tensor."""
+    if codes is None and scales is None:
+        done = fast().tokenwise_quantize(x, bits)
+        if done is not None:
+            return done
     _require_cuda(x, codes, scales)
     _check_flat(x)
     if bits not in (8, 4):

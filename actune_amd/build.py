@@ -23,6 +23,9 @@ SOURCES = ["api.hip", "quantize.hip", "gemm_smallm.hip", "gemm_wide_w2.hip", "ge
 # diagnostic library of register-resident compute ceilings, timed by bench.py
 CEILING_SOURCE = "ceiling.hip"
 CEILING_LIB = LIB_DIR / "libactune_ceiling.so"
+# native call path of the Python modules (host code against torch's headers)
+BINDING_SOURCE = "binding.cpp"
+BINDING_LIB = LIB_DIR / "_actune_fast.so"
 ARCH = "gfx950"
 
 
@@ -79,12 +82,33 @@ def _compile(src: str, incremental: bool = False) -> Path:
     return out
 
 
+def _build_binding(incremental: bool = False) -> None:
+    if incremental and not _stale(BINDING_SOURCE, BINDING_LIB):
+        return
+    import sysconfig
+
+    import torch
+    root = Path(torch.__file__).parent
+    include = [root / "include", root / "include/torch/csrc/api/include", Path(hipcc()).resolve().parents[1] / "include",
+               Path(sysconfig.get_paths()["include"])]
+    tmp = BINDING_LIB.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{p}" for p in include),
+           str(CSRC / BINDING_SOURCE), "-o", str(tmp), f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu",
+           "-ltorch_hip", "-ltorch", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode:
+        raise RuntimeError(f"g++ failed for {BINDING_SOURCE}:\n{res.stderr}")
+    os.replace(tmp, BINDING_LIB)
+
+
 def build(verbose: bool = False, incremental: bool = False) -> Path:
     """Compile every source (or, incremental, only the out-of-date ones) and
     link the library."""
     OBJ.mkdir(exist_ok=True)
     LIB_DIR.mkdir(exist_ok=True)
-    with concurrent.futures.ThreadPoolExecutor(max_workers=len(SOURCES) + 1) as pool:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=len(SOURCES) + 2) as pool:
+        binding = pool.submit(_build_binding, incremental)
         objs = list(pool.map(lambda src: _compile(src, incremental), SOURCES + [CEILING_SOURCE]))
     for lib, parts in ((LIB, objs[:-1]), (CEILING_LIB, objs[-1:])):
         tmp = lib.with_suffix(".so.tmp")
@@ -93,6 +117,7 @@ def build(verbose: bool = False, incremental: bool = False) -> Path:
         if res.returncode:
             raise RuntimeError(f"link failed:\n{res.stderr}")
         os.replace(tmp, lib)
+    binding.result()
     if verbose:
         print(f"built {LIB}", file=sys.stderr)
     return LIB

@@ -202,6 +202,10 @@ def _split_workspace(m, n, k, w_layout, a_layout, device, targets=1):
 
 
 def _gemm(activation, a_layout, scale, weight, w_layout, weight_scale, bias, n, k, epilogue, dtype):
+    done = _native.fast().tokenwise_linear(activation, a_layout, scale, weight, w_layout, weight_scale, bias, n, k,
+                                           epilogue, _native.DTYPE_CODES.get(dtype, -1))
+    if done is not None:
+        return done
     out = torch.empty((activation.shape[0], n), device=activation.device, dtype=dtype)
     ws = _split_workspace(activation.shape[0], n, k, w_layout, a_layout, activation.device)
     return _native.tokenwise_linear(activation, a_layout, scale, weight, w_layout, weight_scale, bias, n, k,
@@ -425,6 +429,10 @@ class _TokenwiseA8(torch.nn.Module):
         m = flat.shape[0]
         weight, wscale, bias, n = _kernel_operands(self, getattr(self, self._weight_name), self.bias)
         if self._fuses_rows(flat):
+            done = _native.fast().tokenwise_linear_x(flat.contiguous(), weight, self._layout, wscale, bias, n,
+                                                     self.in_features, _native.TW_EPI_A8)
+            if done is not None:
+                return _first_columns(done, self.out_features).reshape(*original_shape, self.out_features)
             out = torch.empty((m, n), device=flat.device, dtype=value.dtype)
             scale = torch.empty(m, device=flat.device, dtype=torch.float32)
             ws = _split_workspace(m, n, self.in_features, self._layout, _native.TW_ACT_A8, flat.device)
@@ -760,16 +768,18 @@ def _record(issue, device):
 
 
 class DecodeGraphPlan:
-    """A captured decode of 1 to 4 sibling projections of one row (K-major
+    """A prepared decode of 1 to 4 sibling projections of one row (K-major
     W4, each with an optional signed R4 residual). The contract is the
-    reference's (decode_w4a8_triton.py:326-425): each run
-    copies the row into the plan's staging buffer, replays, and returns the
-    outputs [projections, N] as a fresh tensor, so callers never hold
-    graph-owned memory. The graph holds two launches: the GEMM over every
-    projection's tiles that quantizes the row itself (rows up to 16384
-    long; longer rows add the quantizer launch first) and the integer reduce
-    for all projections. Runs are serialised by a lock, since they share the
-    staging buffers."""
+    reference's (decode_w4a8_triton.py:326-425): each run takes a row and
+    returns the outputs [projections, N] as a fresh tensor, so callers never
+    hold plan-owned memory. Rows up to 16384 long take two launches, issued
+    directly: the GEMM over every projection's tiles, which quantizes the row
+    itself, and the integer reduce for all projections. (Replaying a graph of
+    the two took 16 us of host time and a copy of the row in and of the
+    outputs out, 34 us a run; issued directly, about 9.) Longer rows add the
+    quantizer launch and replay a graph of the three between staging buffers;
+    those runs are serialised by a lock. ``graph_replays`` counts the runs of
+    either form."""
 
     def __init__(self, value, weights, residuals, scales, biases):
         if not 1 <= len(weights) <= _native.MAX_TARGETS:
@@ -779,41 +789,61 @@ class DecodeGraphPlan:
         self.n, self.k = _w4_shape(self.weights[0])
         self.groups = len(self.weights)
         self.layout = _decode_layout(self.residuals)
-        dev = value.device
+        self.device, self.dtype = value.device, value.dtype
         self.quantize_in_gemm = self.k <= _FUSED_MAX_K
+        self.lock = threading.Lock()
+        if self.quantize_in_gemm:
+            self._held = ()
+            self._direct(value)  # runs every argument check
+            return
+        dev = value.device
         self.input = torch.empty((1, self.k), device=dev, dtype=value.dtype)
-        self.activation = None if self.quantize_in_gemm else torch.empty((1, self.k), device=dev, dtype=torch.int8)
+        self.activation = torch.empty((1, self.k), device=dev, dtype=torch.int8)
         self.scale = torch.empty(1, device=dev, dtype=torch.float32)
         self.output = torch.empty((self.groups, self.n), device=dev, dtype=value.dtype)
         need = self.groups * _native.tokenwise_workspace_bytes(1, self.n, self.k, self.layout, _native.TW_ACT_A8)
         self.partial = torch.empty(need, device=dev, dtype=torch.uint8) if need else None
-        self.lock = threading.Lock()
+        self._held = (self.input, self.activation, self.scale, self.output, self.partial)
         self.input.copy_(value.reshape(1, self.k))
         self.graph = _record(self._issue, dev)
 
+    def _targets(self, output):
+        return [(w, s, b, output[i:i + 1])
+                for i, (w, s, b) in enumerate(zip(self.weights, self.scales, self.biases))]
+
+    def _direct(self, value):
+        row = _native._aligned16(value.reshape(1, self.k).to(self.device, self.dtype).contiguous())
+        done = _native.fast().tokenwise_decode(row, self.weights, self.residuals, self.scales, self.biases,
+                                               self.layout, self.n, self.k, _native.TW_EPI_A8)
+        if done is not None:
+            return done
+        output = torch.empty((self.groups, self.n), device=self.device, dtype=self.dtype)
+        _native.tokenwise_linear_multi(
+            self._targets(output), self.layout, self.n, self.k, _native.TW_EPI_A8,
+            torch.empty(1, device=self.device, dtype=torch.float32), x=row,
+            workspace=_split_workspace(1, self.n, self.k, self.layout, _native.TW_ACT_A8, self.device, self.groups),
+            residuals=self.residuals if self.layout == _native.TW_KMAJOR_W4R4 else None)
+        return output
+
     def _issue(self):
-        targets = [(w, s, b, self.output[i:i + 1])
-                   for i, (w, s, b) in enumerate(zip(self.weights, self.scales, self.biases))]
         residuals = self.residuals if self.layout == _native.TW_KMAJOR_W4R4 else None
-        if self.quantize_in_gemm:
-            _native.tokenwise_linear_multi(targets, self.layout, self.n, self.k, _native.TW_EPI_A8, self.scale,
-                                           x=self.input, workspace=self.partial, residuals=residuals)
-        else:
-            _native.tokenwise_quantize(self.input, 8, self.activation, self.scale)
-            _native.tokenwise_linear_multi(targets, self.layout, self.n, self.k, _native.TW_EPI_A8, self.scale,
-                                           codes=self.activation, workspace=self.partial, residuals=residuals)
+        _native.tokenwise_quantize(self.input, 8, self.activation, self.scale)
+        _native.tokenwise_linear_multi(self._targets(self.output), self.layout, self.n, self.k, _native.TW_EPI_A8,
+                                       self.scale, codes=self.activation, workspace=self.partial, residuals=residuals)
 
     @property
     def workspace_bytes(self):
         """Device bytes the plan holds outside the graph's own pool."""
-        held = (self.input, self.activation, self.scale, self.output, self.partial)
-        return sum(t.numel() * t.element_size() for t in held if t is not None)
+        return sum(t.numel() * t.element_size() for t in self._held if t is not None)
 
     def run(self, value):
-        with self.lock:
-            self.input.copy_(value.reshape(1, self.k))
-            self.graph.replay()
-            result = self.output.clone()
+        if self.quantize_in_gemm:
+            result = self._direct(value)
+        else:
+            with self.lock:
+                self.input.copy_(value.reshape(1, self.k))
+                self.graph.replay()
+                result = self.output.clone()
         separate = int(not self.quantize_in_gemm)
         _count(1, graph_replays=1, graph_quantization_kernels=separate, resident_quantization_kernels=separate)
         _count_split_decode(self.groups, self.n, self.k, self.layout)
