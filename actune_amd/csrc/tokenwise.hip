@@ -24,8 +24,9 @@
 //   A8 family: t = f32(acc) * as[m]; y = bias ? fmaf(t, ws[n], bias[n]) : t * ws[n]
 //   native A4: q = as[m] * ws[n];    y = bias ? fmaf(f32(acc), q, bias[n]) : f32(acc) * q
 //
-// MFMA operands (v_mfma_i32_16x16x64_i8): tokens are the A operand, output
-// channels the B operand; lane l holds row l % 16 and the 16 k-slots of
+// MFMA operands (v_mfma_i32_16x16x64_i8): output channels are the A operand,
+// tokens the B operand, so that a lane's four results are consecutive
+// channels of one token; lane l holds row l % 16 and the 16 k-slots of
 // group kb = l / 16. The k index behind each slot only has to be the same
 // for both operands, so each weight layout uses the slot order its bytes
 // give cheapest:
@@ -44,6 +45,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "../../include/actune_hip.h"
 #include "common.hpp"
@@ -163,60 +165,135 @@ __device__ __forceinline__ TwArgs for_target(const TwArgs& in, int i) {
   return a;
 }
 
-// y for output (m, n) from the true int32 accumulator, in the family's
-// fixed fp32 sequence, stored in out_dt.
-template <int EPI>
-__device__ __forceinline__ void store_result(const TwArgs& a, int m, int n, int32_t acc) {
-  const float x = (float)acc;
-  const float as = a.as[m], ws = a.ws[n] * a.ws_mul;
-  float y;
-  if constexpr (EPI == ACTUNE_TW_EPI_A8) {
-    const float t = x * as;
-    y = a.bias ? __builtin_fmaf(t, ws, load_bias(a.bias, a.bias_dt, n)) : t * ws;
-  } else {
-    const float q = as * ws;
-    y = a.bias ? __builtin_fmaf(x, q, load_bias(a.bias, a.bias_dt, n)) : x * q;
-  }
-  const size_t o = (size_t)m * a.N + n;
-  if (a.out_dt == kBF16) store_out<kBF16>(a.out, o, y);
-  else if (a.out_dt == kF16) store_out<kF16>(a.out, o, y);
-  else store_out<kF32>(a.out, o, y);
+// Scales and biases of C consecutive columns from n (columns past N: zeros).
+template <int C>
+struct TwCols {
+  float ws[C], bias[C];
+};
+
+template <int DT, int C, int NT>
+__device__ __forceinline__ void load_bias_cols(const TwArgs& a, int n, TwCols<C> (&c)[NT]) {
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int r = 0; r < C; ++r) {
+      const int at = n + 16 * nt + r;
+      c[nt].bias[r] = at < a.N ? load_as_f32<DT>(a.bias, at) : 0.f;
+    }
 }
 
-// Writes a wave's MT x NT accumulator tiles (lane: rows row_base + 16 mt +
-// 0..3, column col_base + 16 nt): with K splits, split z's raw int32 partial
-// sums (tw_reduce adds the splits, in any order, and finishes); otherwise
-// the finished outputs.
+// column groups n, n + 16, ... n + 16 (NT - 1): every load is issued before
+// the first is used
+template <int C, int NT>
+__device__ __forceinline__ void load_cols(const TwArgs& a, int n, TwCols<C> (&c)[NT]) {
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int r = 0; r < C; ++r) {
+      const int at = n + 16 * nt + r;
+      c[nt].ws[r] = (at < a.N ? a.ws[at] : 0.f) * a.ws_mul;
+      c[nt].bias[r] = 0.f;
+    }
+  if (!a.bias) return;
+  if (a.bias_dt == kBF16) load_bias_cols<kBF16>(a, n, c);
+  else if (a.bias_dt == kF16) load_bias_cols<kF16>(a, n, c);
+  else load_bias_cols<kF32>(a, n, c);
+}
+
+// y of C columns of row m from the true int32 accumulators, in the family's
+// fixed fp32 sequence, stored in DT: one store where `wide` (four columns,
+// all inside N, on their alignment), otherwise one per column inside N.
+template <int EPI, int DT, int C>
+__device__ __forceinline__ void store_cols(const TwArgs& a, int m, int n, float as, const TwCols<C>& c,
+                                           const int32_t (&acc)[C], bool wide) {
+  float y[C];
+#pragma unroll
+  for (int r = 0; r < C; ++r) {
+    const float x = (float)acc[r];
+    if constexpr (EPI == ACTUNE_TW_EPI_A8) {
+      const float t = x * as;
+      y[r] = a.bias ? __builtin_fmaf(t, c.ws[r], c.bias[r]) : t * c.ws[r];
+    } else {
+      const float q = as * c.ws[r];
+      y[r] = a.bias ? __builtin_fmaf(x, q, c.bias[r]) : x * q;
+    }
+  }
+  const size_t o = (size_t)m * a.N + n;
+  if constexpr (C == 4) {
+    if (wide) {
+      if constexpr (DT == kF32) {
+        *reinterpret_cast<v4f*>((float*)a.out + o) = v4f{y[0], y[1], y[2], y[3]};
+      } else {
+        uint32_t h[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) h[r] = DT == kBF16 ? f32_to_bf16(y[r]) : f32_to_f16(y[r]);
+        *reinterpret_cast<v2u*>((uint16_t*)a.out + o) = v2u{h[0] | h[1] << 16, h[2] | h[3] << 16};
+      }
+      return;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < C; ++r)
+    if (n + r < a.N) store_out<DT>(a.out, o + r, y[r]);
+}
+
+__device__ __forceinline__ bool wide_rows(const void* out, int dt, int N) {
+  return N % 4 == 0 && (uintptr_t)out % (dt == kF32 ? 16 : 8) == 0;
+}
+
+// Writes a wave's MT x NT accumulator tiles (lane: row `row` + 16 mt, columns
+// `col` + 16 nt + 0..3): with K splits, split z's raw int32 partial sums
+// (tw_reduce adds the splits, in any order, and finishes); otherwise the
+// finished outputs. The scales are loaded ahead of every use and the output
+// type is chosen once: loading and choosing per output had put a memory round
+// trip behind each of a lane's 32 to 64 outputs (128 x 128 tiles of 512 x
+// 4096 x 4096 W4A4: 41 us, 29 now).
 template <int WL, int AL, int EPI, int MT, int NT>
-__device__ __forceinline__ void finish_tile(const TwArgs& args, const v4i (&acc)[MT][NT], int row_base,
-                                            int col_base, int z) {
+__device__ __forceinline__ void finish_tile(const TwArgs& args, const v4i (&acc)[MT][NT], int row, int col, int z) {
   constexpr int SHIFT = WTraits<WL>::TW + (AL == ACTUNE_TW_ACT_A4 ? 4 : 0);
   const int M = args.M, N = args.N;
   if (args.splits > 1) {
     int32_t* part = args.partial + (size_t)z * M * N;
+    const bool wide = wide_rows(part, kF32, N);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
+      for (int nt = 0; nt < NT; ++nt) {
+        const int m = row + mt * 16, n = col + nt * 16;
+        if (m >= M || n >= N) continue;
+        int32_t* p = part + (size_t)m * N + n;
+        if (wide) {
+          *reinterpret_cast<v4i*>(p) = acc[mt][nt];
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int m = row_base + mt * 16 + i, n = col_base + nt * 16;
-          if (m < M && n < N) part[(size_t)m * N + n] = acc[mt][nt][i];
+          for (int r = 0; r < 4; ++r)
+            if (n + r < N) p[r] = acc[mt][nt][r];
         }
+      }
     return;
   }
+  float as[MT];
+  TwCols<4> cols[NT];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int n = col_base + nt * 16;
-    if (n >= N) continue;
+  for (int mt = 0; mt < MT; ++mt) as[mt] = row + mt * 16 < M ? args.as[row + mt * 16] : 0.f;
+  load_cols(args, col, cols);
+  const bool wide = wide_rows(args.out, args.out_dt, N);
+  auto emit = [&](auto dt) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = row_base + mt * 16 + i;
-        if (m < M) store_result<EPI>(args, m, n, acc[mt][nt][i] >> SHIFT);
+      for (int nt = 0; nt < NT; ++nt) {
+        const int m = row + mt * 16, n = col + nt * 16;
+        if (m >= M || n >= N) continue;
+        int32_t x[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = acc[mt][nt][r] >> SHIFT;
+        store_cols<EPI, decltype(dt)::value>(args, m, n, as[mt], cols[nt], x, wide);
       }
-  }
+  };
+  if (args.out_dt == kBF16) emit(std::integral_constant<int, kBF16>{});
+  else if (args.out_dt == kF16) emit(std::integral_constant<int, kF16>{});
+  else emit(std::integral_constant<int, kF32>{});
 }
 
 // Bytes of 16 q4 + r4 as int8, wrapped to 8 bits (decode_w4a8_triton.py:61-66
@@ -452,7 +529,7 @@ __global__ __launch_bounds__(kThreads) void tw_gemm(const TwArgs args_in) {
           else if constexpr (WL == ACTUNE_TW_ROWS_S2) reorder_slot<8, 2>(af);
         }
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = mfma16x16x64(af, bf[nt], acc[mt][nt]);
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = mfma16x16x64(bf[nt], af, acc[mt][nt]);
       }
     }
   };
@@ -650,7 +727,7 @@ __global__ __launch_bounds__(kThreads) void tw_gemm(const TwArgs args_in) {
 #pragma unroll
   for (int i = 0; i < NB; ++i) compute(i);
 
-  finish_tile<WL, AL, EPI, MT, NT>(fin, acc, m0 + wm * 16 * MT + 4 * kb, n0 + wn * 16 * NT + r16, z);
+  finish_tile<WL, AL, EPI, MT, NT>(fin, acc, m0 + wm * 16 * MT + r16, n0 + wn * 16 * NT + 4 * kb, z);
 }
 
 // ------------------------------------------------------------ LDS-DMA ring
@@ -688,6 +765,22 @@ __device__ __forceinline__ constexpr int lds_pos(int r, int b) {
   return r * RB + 16 * ((b >> 4) ^ swz<RB>(r)) + (b & 15);
 }
 
+// The tile (column, row) of a ring workgroup. Workgroups go to the 8 XCDs in
+// turn, each with its own L2: an XCD takes a contiguous eighth of the tiles,
+// counted down columns of 8 tile rows, so that the workgroups it holds at a
+// time form a near-square block and share its weight and activation tiles
+// (1500 x 11008 x 4096 W8A8: 147 us in row order, 138 in this one).
+__device__ __forceinline__ int2 ring_tile() {
+  constexpr int kXcds = 8, kRows = 8;
+  const int cols = (int)gridDim.x, rows = (int)gridDim.y, total = cols * rows;
+  const int id = (int)blockIdx.x + cols * (int)blockIdx.y;
+  const int xcd = id % kXcds;
+  const int t = xcd * (total / kXcds) + min(xcd, total % kXcds) + id / kXcds;
+  const int first = t / (kRows * cols) * kRows, high = min(kRows, rows - first);
+  const int in = t - first * cols;
+  return make_int2(in / high, first + in % high);
+}
+
 // Large-M tokenwise GEMM: the tile geometry of tw_gemm, with the K-steps
 // staged through a ring of D LDS slots filled by DMA loads; a slot holds KS
 // consecutive K-steps (one ring step). Every K-step of a workgroup is NI
@@ -716,7 +809,8 @@ __global__ __launch_bounds__(kThreads) void tw_gemm_ring(const TwArgs args_in) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
-  const int n0 = (int)blockIdx.x * TN, m0 = (int)blockIdx.y * TM;
+  const int2 tile = ring_tile();
+  const int n0 = tile.x * TN, m0 = tile.y * TM;
   const int z = (int)blockIdx.z % args.splits;
   const int g0 = (int)((long)z * args.steps / args.splits), g1 = (int)((long)(z + 1) * args.steps / args.splits);
 
@@ -916,7 +1010,7 @@ __global__ __launch_bounds__(kThreads) void tw_gemm_ring(const TwArgs args_in) {
             unpack_slot<2>(&pw, bf);
           }
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) acc[mt][nt] = mfma16x16x64(af[mt], bf, acc[mt][nt]);
+          for (int mt = 0; mt < MT; ++mt) acc[mt][nt] = mfma16x16x64(bf, af[mt], acc[mt][nt]);
         }
       }
     }
@@ -970,7 +1064,7 @@ __global__ __launch_bounds__(kThreads) void tw_gemm_ring(const TwArgs args_in) {
   }
   // no DMA may still be writing this workgroup's LDS when it ends
   wait_vmem<0>();
-  finish_tile<WL, AL, EPI, MT, NT>(args, acc, m0 + wm * 16 * MT + 4 * kb, n0 + wn * 16 * NT + r16, z);
+  finish_tile<WL, AL, EPI, MT, NT>(args, acc, m0 + wm * 16 * MT + r16, n0 + wn * 16 * NT + 4 * kb, z);
 }
 
 // Adds the K splits' partial sums and finishes the outputs of target
@@ -991,8 +1085,12 @@ __global__ __launch_bounds__(kThreads) void tw_reduce(const TwArgs args_in, int 
   const uint32_t total = (uint32_t)M * (uint32_t)N;
   const Rsrc pr = make_rsrc(args.partial, (uint32_t)S * total * 4u);
   const bool quads = CPT == 4 && (N & 3) == 0;
+  const bool wide = CPT == 4 && wide_rows(args.out, args.out_dt, N);
+  TwCols<CPT> cols[1];
+  load_cols(args, n0, cols);
   for (int m = (int)blockIdx.y; m < M; m += (int)gridDim.y) {
     const uint32_t base = (uint32_t)m * (uint32_t)N + (uint32_t)n0;
+    const float as = args.as[m];
     int32_t sum[CPT] = {};
     for (int s0 = 0; s0 < S; s0 += NS) {
       int32_t v[NS][CPT];
@@ -1018,8 +1116,10 @@ __global__ __launch_bounds__(kThreads) void tw_reduce(const TwArgs args_in, int 
         for (int r = 0; r < CPT; ++r) sum[r] += v[j][r];
     }
 #pragma unroll
-    for (int r = 0; r < CPT; ++r)
-      if (n0 + r < N) store_result<EPI>(args, m, n0 + r, sum[r] >> shift);
+    for (int r = 0; r < CPT; ++r) sum[r] >>= shift;
+    if (args.out_dt == kBF16) store_cols<EPI, kBF16>(args, m, n0, as, cols[0], sum, wide);
+    else if (args.out_dt == kF16) store_cols<EPI, kF16>(args, m, n0, as, cols[0], sum, wide);
+    else store_cols<EPI, kF32>(args, m, n0, as, cols[0], sum, wide);
   }
 }
 
@@ -1114,20 +1214,48 @@ int64_t tiles_of(int64_t M, int64_t N, const Geometry& g) {
 }
 
 // M <= 32: 16-row x 128-column tiles, every K-step of a workgroup loaded at
-// entry (small_ns; tw_gemm). Larger M: the LDS-DMA ring (tw_gemm_ring),
-// chosen from measurements on MI355X at M = 512 over the Llama-2-7B shapes
-// (six layout pairs): where the 64 x 128 grid holds at least 512 tiles (two or
-// more workgroups per CU), 64 x 128 tiles with 3 slots of one K-step (two for
-// the row-major S4 / S2 layouts), small enough in LDS for three workgroups
-// per CU (W4A8 11008x4096: 60.8 -> 45.9 us); with fewer tiles, 4 slots of two
-// K-steps, on 64 x 128 tiles for the K-major layouts and 64 x 64 tiles for S4
-// / S2 (W4A8 4096x11008: 57.7 -> 51.2 us, W4A4 4096x4096: 30.4 -> 20.3 us).
+// entry (small_ns; tw_gemm). Larger M: the LDS-DMA ring (tw_gemm_ring). Tile
+// counts below are of its 64 x 128 tile.
+//
+// Up to 256 tiles, one per CU: 4 slots of two K-steps, so that one workgroup
+// alone keeps enough bytes in flight (512 x 4096 x 4096 W8A8, quantizer
+// included: 18.8 us, 26.4 us with 3 slots of one), on 64 x 64 tiles for the
+// row-major layouts. Up to 511, two per CU: what leaves LDS for two, 3 slots
+// of two K-steps for W8 and the row-major layouts (300 x 11008 x 4096 W8A8:
+// 26.8 us, 33.9 with 4 slots, 32.5 with one K-step), 4 of two for the nibble
+// pairs (26.7; 30.7 with 3 of one), 3 of one for the quarters, whose
+// activation tile is twice as wide (25.1; 34.8).
+//
+// From 512 on the grid runs in rounds of one tile per CU, with two or three
+// in flight, and a tile of 96, 128 or (W8) 192 rows reads fewer weight bytes
+// and reads LDS less often per product, so that its round takes 1.2, 1.5 and
+// 2.3 times as long as a 64-row round (in the layouts that unpack the weight
+// tile from K-major fields 1.4 and 2), measured over M = 500-2000 on
+// six layouts. The fewest rounds by that weight win: 1500 x 11008 x 4096
+// W8A8 123 us at 64 rows, 90 at 96, 97 at 128, 83 at 192 (taken); 2000 x 4096
+// x 4096 W8A8 52, 47, 43 (taken), 50; 1500 x 11008 x 4096 W4A4 111, 85
+// (taken), 91.
 Geometry pick_geometry(int64_t M, int64_t N, int wl) {
   if (M <= 32) return Geometry{1, 1, 2, small_ns(wl), 0, 0};
-  const bool km = kmajor(wl);
-  const Geometry big{2, 2, 4, 0, km ? 1 : 2, 3};
-  if (tiles_of(M, N, big) >= 512) return big;
-  return km ? Geometry{2, 2, 4, 0, 2, 4} : Geometry{2, 2, 2, 0, 2, 4};
+  const bool km = kmajor(wl), w8 = wl == ACTUNE_TW_KMAJOR_W8;
+  const int ks = km ? 1 : 2;
+  const Geometry base{2, 2, 4, 0, ks, 3}, deep{2, 2, 4, 0, 2, 4};
+  const int64_t tiles = tiles_of(M, N, base);
+  if (tiles <= 256) return km ? deep : Geometry{2, 2, 2, 0, 2, 4};
+  if (tiles < 512) {
+    if (wl == ACTUNE_TW_KMAJOR_W4) return deep;
+    return wl == ACTUNE_TW_KMAJOR_W2 ? base : Geometry{2, 2, 4, 0, 2, 3};
+  }
+  const bool fields = km && !w8;
+  const Geometry sizes[4] = {base, {2, 3, 4, 0, ks, 3}, {2, 4, 4, 0, ks, km ? 4 : 3}, {2, 6, 4, 0, ks, 4}};
+  const int round[4] = {fields ? 10 : 11, fields ? 14 : 13, fields ? 20 : 17, 25};
+  int best = 0;
+  int64_t least = INT64_MAX;
+  for (int i = 0; i < (w8 ? 4 : 3); ++i) {
+    const int64_t t = round[i] * ((tiles_of(M, N, sizes[i]) + 255) / 256);
+    if (t < least) least = t, best = i;
+  }
+  return sizes[best];
 }
 
 // K splits. Small M: the fewest splits whose ranges fit a workgroup's entry
@@ -1215,9 +1343,22 @@ void launch_gemm_g(const TwArgs& a, const Geometry& g, hipStream_t st) {
     launch_gemm_t<WL, AL, EPI, 1, 1, 2, 4>(a, st);
   } else {
     if (g.wm == 1) launch_gemm_t<WL, AL, EPI, 1, 1, 2, (WL == ACTUNE_TW_KMAJOR_W8 ? 4 : 8)>(a, st);
-    else if (g.d == 3) launch_ring_t<WL, AL, EPI, 2, 2, 4, KM ? 1 : 2, 3>(a, st);
-    else if constexpr (KM) launch_ring_t<WL, AL, EPI, 2, 2, 4, 2, 4>(a, st);
-    else launch_ring_t<WL, AL, EPI, 2, 2, 2, 2, 4>(a, st);
+    else if (g.mt == 2 && g.nt == 2) {
+      if constexpr (!KM) launch_ring_t<WL, AL, EPI, 2, 2, 2, 2, 4>(a, st);
+    } else if (g.mt == 2 && g.d == 4) {
+      if constexpr (KM) launch_ring_t<WL, AL, EPI, 2, 2, 4, 2, 4>(a, st);
+    } else if (g.mt == 2) {
+      if constexpr (!KM || WL == ACTUNE_TW_KMAJOR_W8) {
+        if (g.ks == 2) return launch_ring_t<WL, AL, EPI, 2, 2, 4, 2, 3>(a, st);
+      }
+      if constexpr (KM) launch_ring_t<WL, AL, EPI, 2, 2, 4, 1, 3>(a, st);
+    } else if (g.mt == 3) {
+      launch_ring_t<WL, AL, EPI, 2, 3, 4, KM ? 1 : 2, 3>(a, st);
+    } else if (g.mt == 4) {
+      launch_ring_t<WL, AL, EPI, 2, 4, 4, KM ? 1 : 2, KM ? 4 : 3>(a, st);
+    } else {
+      if constexpr (WL == ACTUNE_TW_KMAJOR_W8) launch_ring_t<WL, AL, EPI, 2, 6, 4, 1, 4>(a, st);
+    }
   }
 }
 
