@@ -362,22 +362,16 @@ def grouped_linear(a, as_, w, ws, bias, source_or_shape, W, A, config=CONFIG_AUT
     packed activations + scales x packed weights -> [M, N] in source.dtype.
     ``source_or_shape`` is the [M, K] source tensor (its dtype and shape
     define the output), as in the reference op signature."""
-    if out is None:
-        if isinstance(source_or_shape, torch.Tensor):
-            shape, dtype = source_or_shape.shape, source_or_shape.dtype
-        else:
-            shape, dtype = source_or_shape, out_dtype or torch.bfloat16
-        if len(shape) == 2:
-            done = fast().grouped_linear(a, as_, w, ws, bias, *shape, DTYPE_CODES.get(dtype, -1), W, A, config)
-            if done is not None:
-                return done
-    _require_cuda(a, as_, w, ws, bias)
     if isinstance(source_or_shape, torch.Tensor):
-        m, k = source_or_shape.shape
-        dtype = source_or_shape.dtype
+        shape, dtype = source_or_shape.shape, source_or_shape.dtype
     else:
-        m, k = source_or_shape
-        dtype = out_dtype or torch.bfloat16
+        shape, dtype = tuple(source_or_shape), out_dtype or torch.bfloat16
+    if out is None and len(shape) == 2:
+        done = fast().grouped_linear(a, as_, w, ws, bias, *shape, DTYPE_CODES.get(dtype, -1), W, A, config)
+        if done is not None:
+            return done
+    _require_cuda(a, as_, w, ws, bias)
+    m, k = shape
     n = w.size(0)
     if W not in (2, 4, 8) or A not in (2, 4, 8):
         raise ValueError("Unsupported integer width")

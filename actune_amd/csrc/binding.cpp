@@ -6,10 +6,10 @@
 // allocations, the current stream and seventeen converted arguments. Each
 // function here takes the plain case of one of its calls: every operand on
 // one GPU, contiguous, of the expected type and shape, 16-byte aligned, no
-// caller-owned buffers. Anything else returns None, and the ctypes path, which
-// names what is wrong or makes an aligned copy, takes the call. Output and
-// scratch come from torch's caching allocator on the current stream, as
-// there; nothing is kept between calls.
+// caller-owned buffers. Anything else, an argument of another type included,
+// returns None, and the ctypes path, which names what is wrong or makes an
+// aligned copy, takes the call. Output and scratch come from torch's caching
+// allocator on the current stream, as there; nothing is kept between calls.
 #include <torch/extension.h>
 
 #include <c10/hip/HIPStream.h>
@@ -134,7 +134,8 @@ py::object grouped_linear(const Tensor& a, const Tensor& as, const Tensor& w, co
   if (!a.is_cuda() || !width_ok(W) || !width_ok(A) || k <= 0 || k % 64 || out_code < 0) return py::none();
   const at::Device dev = a.device();
   if (!plain(a, dev, at::kByte) || a.dim() != 2 || a.size(0) != m || a.size(1) != k * A / 8 || !plain(as, dev, at::kFloat) ||
-      as.dim() != 2 || as.size(0) != m || as.size(1) != k / 64 || !weights_ok(w, ws, bias, dev, k, W))
+      as.dim() != 2 || as.size(0) != m || as.size(1) != k / 64 || !weights_ok(w, ws, bias, dev, k, W) ||
+      w.size(0) == 0)
     return py::none();
   const int64_t n = w.size(0);
   Tensor out = empty({m, n}, dev, dtype_of(out_code));
@@ -149,8 +150,10 @@ py::object grouped_linear(const Tensor& a, const Tensor& as, const Tensor& w, co
   return py::cast(out);
 }
 
-// targets: (w, w_scale, bias or None, None[, W])
-py::object grouped_forward_multi(const Tensor& x, const std::vector<py::tuple>& targets, int64_t W, int64_t A,
+bool is_tensor(const py::object& o) { return THPVariable_Check(o.ptr()); }
+
+// targets: sequences (w, w_scale, bias or None, None[, W])
+py::object grouped_forward_multi(const Tensor& x, const py::sequence& targets, int64_t W, int64_t A,
                                  const OptTensor& scale, int config) {
   const size_t count = targets.size();
   if (count < 1 || count > ACTUNE_MAX_TARGETS || !rows_ok(x) || !width_ok(W) || !width_ok(A) || x.size(1) <= 0 ||
@@ -160,19 +163,29 @@ py::object grouped_forward_multi(const Tensor& x, const std::vector<py::tuple>& 
   const int64_t m = x.size(0), k = x.size(1);
   actune_linear_target t[ACTUNE_MAX_TARGETS];
   std::vector<Tensor> outs;
+  Tensor weights[ACTUNE_MAX_TARGETS], scales[ACTUNE_MAX_TARGETS];  // held over the call (lists can change under it)
+  OptTensor biases[ACTUNE_MAX_TARGETS];
   int bias_type = 2;
   for (size_t i = 0; i < count; ++i) {
-    const py::tuple& g = targets[i];
-    if (g.size() < 4 || !g[3].is_none()) return py::none();
-    const Tensor w = g[0].cast<Tensor>(), ws = g[1].cast<Tensor>();
-    const OptTensor bias = g[2].cast<OptTensor>();
-    const int64_t width = g.size() > 4 ? g[4].cast<int64_t>() : W;
-    if (!width_ok(width) || !weights_ok(w, ws, bias, dev, k, width)) return py::none();
+    const py::object target = targets[i];
+    if (!PyTuple_Check(target.ptr()) && !PyList_Check(target.ptr())) return py::none();
+    const auto g = py::reinterpret_borrow<py::sequence>(target);
+    const size_t fields = g.size();
+    if (fields < 4) return py::none();
+    const py::object gw = g[0], gs = g[1], gb = g[2], go = g[3], gn = fields > 4 ? py::object(g[4]) : py::none();
+    if (!is_tensor(gw) || !is_tensor(gs) || !(gb.is_none() || is_tensor(gb)) || !go.is_none() ||
+        !(fields < 5 || PyLong_Check(gn.ptr())))
+      return py::none();
+    const Tensor &w = weights[i] = gw.cast<Tensor>(), &scale_w = scales[i] = gs.cast<Tensor>();
+    const OptTensor& bias = biases[i] = gb.cast<OptTensor>();
+    int overflow = 0;
+    const int64_t width = fields > 4 ? PyLong_AsLongLongAndOverflow(gn.ptr(), &overflow) : W;
+    if (overflow || !width_ok(width) || !weights_ok(w, scale_w, bias, dev, k, width)) return py::none();
     const bool same = i == 0 || ((t[0].bias != nullptr) == bias.has_value() && bias_type == bias_code(bias));
     if (!same) return py::none();
     bias_type = bias_code(bias);
     outs.push_back(empty({m, w.size(0)}, dev, x.scalar_type()));
-    t[i] = actune_linear_target{w.const_data_ptr<uint8_t>(), ws.const_data_ptr<float>(), ptr(bias),
+    t[i] = actune_linear_target{w.const_data_ptr<uint8_t>(), scale_w.const_data_ptr<float>(), ptr(bias),
                                 outs[i].mutable_data_ptr(), w.size(0), (int32_t)width};
   }
   const CodeBuffer codes(m, k, A, dev);
@@ -326,15 +339,22 @@ py::object tokenwise_decode(const Tensor& x, const std::vector<Tensor>& weights,
 
 }  // namespace
 
+// A call whose arguments do not convert falls to the second overload.
+template <typename F>
+void def(py::module_& m, const char* name, F f) {
+  m.def(name, f);
+  m.def(name, [](const py::args&) { return py::none(); });
+}
+
 PYBIND11_MODULE(_actune_fast, m) {
   m.def("init", &init);
-  m.def("quantize_groups", &quantize_groups);
-  m.def("quantize_gated", &quantize_gated);
-  m.def("grouped_linear", &grouped_linear);
-  m.def("grouped_forward", &grouped_forward);
-  m.def("grouped_forward_multi", &grouped_forward_multi);
-  m.def("tokenwise_quantize", &tokenwise_quantize);
-  m.def("tokenwise_linear", &tokenwise_linear);
-  m.def("tokenwise_linear_x", &tokenwise_linear_x);
-  m.def("tokenwise_decode", &tokenwise_decode);
+  def(m, "quantize_groups", &quantize_groups);
+  def(m, "quantize_gated", &quantize_gated);
+  def(m, "grouped_linear", &grouped_linear);
+  def(m, "grouped_forward", &grouped_forward);
+  def(m, "grouped_forward_multi", &grouped_forward_multi);
+  def(m, "tokenwise_quantize", &tokenwise_quantize);
+  def(m, "tokenwise_linear", &tokenwise_linear);
+  def(m, "tokenwise_linear_x", &tokenwise_linear_x);
+  def(m, "tokenwise_decode", &tokenwise_decode);
 }

@@ -74,3 +74,41 @@ def test_what_it_does_not_take_behaves_as_before():
             (lambda: N.tokenwise_quantize(rows.clone(), 2), ValueError, "A8 or A4")):
         with pytest.raises(error, match=match):
             bad()
+
+
+def test_arguments_of_another_kind_are_left_to_the_ctypes_path():
+    """Targets may be any sequence of sequences, and an argument of a type that the native call path does not take
+    reaches the checks that name what is wrong."""
+    f = N.fast()
+    x, w, ws = torch.zeros(2, 64, dtype=torch.bfloat16), torch.zeros(4, 32, dtype=torch.uint8), torch.zeros(4)
+    for targets in ([[w, ws, None, None]], ((w, ws, None, None),), [(w, ws, None)], [None], [(None, ws, None, None)],
+                    [(w, ws, 1, None)], [(w, ws, None, None, 4.0)], None, 5):
+        assert f.grouped_forward_multi(x, targets, 4, 8, None, -1) is None
+    for call in (lambda: f.quantize_groups(None, 8, None), lambda: f.quantize_groups(x, 8.0, None),
+                 lambda: f.quantize_gated(x, None, 0, 8, None),
+                 lambda: f.grouped_linear(None, ws, w, ws, None, 2, 64, 0, 4, 8, -1),
+                 lambda: f.grouped_linear(w, ws, w, ws, None, 2.0, 64, 0, 4, 8, -1),
+                 lambda: f.grouped_forward(x, None, ws, None, 4, 8, None, -1),
+                 lambda: f.grouped_forward(x, w, ws, None, 4, 8, None, 2 ** 40), lambda: f.tokenwise_quantize(x, "8"),
+                 lambda: f.tokenwise_linear(None, 0, ws, w, 1, ws, None, 4, 64, 0, 0),
+                 lambda: f.tokenwise_linear_x(x, None, 1, ws, None, 4, 64, 0),
+                 lambda: f.tokenwise_decode(x[:1], [None], [None], [ws], [None], 1, 4, 64, 0)):
+        assert call() is None
+    with pytest.raises(RuntimeError, match="CUDA required"):
+        N.grouped_forward_multi(x, [[w, ws, None, None]], 4, 8)
+    with pytest.raises(RuntimeError, match="CUDA required"):
+        N.grouped_forward_multi(x, [[None, ws, None, None]], 4, 8)
+
+
+@pytest.mark.gpu
+def test_target_sequences_and_empty_outputs():
+    packed, ws = _layer(48, 128, 4)
+    x = torch.randn(4, 128, device=DEV, dtype=torch.bfloat16)
+    want = N.grouped_forward(x, packed, ws, None, 4, 8)
+    for targets in ([[packed, ws, None, None]], ((packed, ws, None, None),), ([packed, ws, None, None, 4],)):
+        assert torch.equal(N.fast().grouped_forward_multi(x, targets, 4, 8, None, -1)[0], want)
+        assert torch.equal(N.grouped_forward_multi(x, targets, 4, 8)[0], want)
+    codes, scales = N.quantize_groups(x, 8)
+    assert torch.equal(N.grouped_linear(codes, scales, packed, ws, None, iter((4, 128)), 4, 8), want)
+    with pytest.raises(RuntimeError, match="invalid dimensions"):
+        N.grouped_linear(codes, scales, packed[:0], ws[:0], None, x, 4, 8)
