@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import importlib.util
+import warnings
 from pathlib import Path
 
 import torch
@@ -83,19 +84,44 @@ _FAST_API = ("actune_quantize_groups", "actune_quantize_gated", "actune_grouped_
              "actune_tokenwise_linear_x", "actune_tokenwise_linear_multi", "actune_last_error")
 
 
+class _CtypesOnly:
+    """Stands in for the native call path where it does not load: takes no
+    call, so that the ctypes path runs each of them."""
+
+    def __getattr__(self, name):
+        if name.startswith("__"):
+            raise AttributeError(name)
+        return lambda *args: None
+
+
+def _load_fast():
+    so = lib()
+    if not FAST_PATH.exists():
+        raise ImportError("it is not built")
+    spec = importlib.util.spec_from_file_location("_actune_fast", FAST_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    if module.torch_version != torch.__version__.split("+")[0]:
+        raise ImportError(f"it was built against torch {module.torch_version}")
+    module.init([ctypes.cast(getattr(so, name), _P).value for name in _FAST_API])
+    return module
+
+
 def fast():
     """The native call path (csrc/binding.cpp) over the loaded library: its
-    functions take the plain case of the calls below, or return None."""
+    functions take the plain case of the calls below, or return None. It only
+    saves host time: where it does not load (not built, or built against
+    another torch or Python) a warning says so, once, and the ctypes path
+    serves every call."""
     global _FAST
     if _FAST is None:
-        so = lib()
-        if not FAST_PATH.exists():
-            raise ImportError(f"{FAST_PATH} is missing: build it with `python -m actune_amd.build`")
-        spec = importlib.util.spec_from_file_location("_actune_fast", FAST_PATH)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        module.init([ctypes.cast(getattr(so, name), _P).value for name in _FAST_API])
-        _FAST = module
+        lib()  # (raises where the kernels themselves are missing)
+        try:
+            _FAST = _load_fast()
+        except ImportError as error:
+            warnings.warn(f"the native call path {FAST_PATH} does not load ({error}): calls take about 10 us more host "
+                          "time; build it with `python -m actune_amd.build`", RuntimeWarning, stacklevel=2)
+            _FAST = _CtypesOnly()
     return _FAST
 
 

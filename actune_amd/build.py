@@ -26,6 +26,7 @@ CEILING_LIB = LIB_DIR / "libactune_ceiling.so"
 # native call path of the Python modules (host code against torch's headers)
 BINDING_SOURCE = "binding.cpp"
 BINDING_LIB = LIB_DIR / "_actune_fast.so"
+BINDING_STAMP = OBJ / "binding.txt"  # the torch and Python it was built against
 ARCH = "gfx950"
 
 
@@ -82,8 +83,28 @@ def _compile(src: str, incremental: bool = False) -> Path:
     return out
 
 
+def cxx() -> str:
+    """The host compiler: $CXX, or g++ or c++ on the PATH."""
+    for cand in (os.environ.get("CXX"), "g++", "c++"):
+        if cand and shutil.which(cand):
+            return cand
+    raise RuntimeError("no host C++ compiler (set CXX); the native call path cannot be built")
+
+
+def _binding_target() -> str:
+    import torch
+    return f"torch {torch.__version__} python {sys.version}"
+
+
+def _binding_stale() -> bool:
+    """True when the extension is out of date, or built against another torch
+    or Python than the ones that run this."""
+    return (_stale(BINDING_SOURCE, BINDING_LIB) or not BINDING_STAMP.exists()
+            or BINDING_STAMP.read_text() != _binding_target())
+
+
 def _build_binding(incremental: bool = False) -> None:
-    if incremental and not _stale(BINDING_SOURCE, BINDING_LIB):
+    if incremental and not _binding_stale():
         return
     import sysconfig
 
@@ -92,14 +113,17 @@ def _build_binding(incremental: bool = False) -> None:
     include = [root / "include", root / "include/torch/csrc/api/include", Path(hipcc()).resolve().parents[1] / "include",
                Path(sysconfig.get_paths()["include"])]
     tmp = BINDING_LIB.with_suffix(".so.tmp")
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{p}" for p in include),
-           str(CSRC / BINDING_SOURCE), "-o", str(tmp), f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu",
-           "-ltorch_hip", "-ltorch", "-ltorch_python"]
+    cmd = [cxx(), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(word for p in include for word in ("-isystem", str(p))), str(CSRC / BINDING_SOURCE), "-o", str(tmp),
+           f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode:
-        raise RuntimeError(f"g++ failed for {BINDING_SOURCE}:\n{res.stderr}")
+        raise RuntimeError(f"{cmd[0]} failed for {BINDING_SOURCE}:\n{res.stderr}")
+    if res.stderr:
+        print(res.stderr, file=sys.stderr)
     os.replace(tmp, BINDING_LIB)
+    BINDING_STAMP.write_text(_binding_target())
 
 
 def build(verbose: bool = False, incremental: bool = False) -> Path:

@@ -13,7 +13,9 @@
 #include <torch/extension.h>
 
 #include <c10/hip/HIPStream.h>
+#include <torch/version.h>
 
+#include <cstring>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -347,6 +349,7 @@ void def(py::module_& m, const char* name, F f) {
 }
 
 PYBIND11_MODULE(_actune_fast, m) {
+  m.attr("torch_version") = TORCH_VERSION;
   m.def("init", &init);
   def(m, "quantize_groups", &quantize_groups);
   def(m, "quantize_gated", &quantize_gated);

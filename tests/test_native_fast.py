@@ -112,3 +112,50 @@ def test_target_sequences_and_empty_outputs():
     assert torch.equal(N.grouped_linear(codes, scales, packed, ws, None, iter((4, 128)), 4, 8), want)
     with pytest.raises(RuntimeError, match="invalid dimensions"):
         N.grouped_linear(codes, scales, packed[:0], ws[:0], None, x, 4, 8)
+
+
+@pytest.mark.parametrize("kind", ["missing", "unloadable", "other torch"])
+def test_calls_run_without_the_extension(kind, monkeypatch, tmp_path):
+    """Without a native call path that loads (none built, or one of another torch) the ctypes path serves every call,
+    after one warning."""
+    path = tmp_path / "_actune_fast.so"
+    if kind == "unloadable":
+        path.write_bytes(b"not a library")
+    elif kind == "other torch":
+        path = N.FAST_PATH
+        monkeypatch.setattr(N.torch, "__version__", "1.0.0")
+    monkeypatch.setattr(N, "FAST_PATH", path)
+    monkeypatch.setattr(N, "_FAST", None)
+    x, w, ws = torch.zeros(2, 64, dtype=torch.bfloat16), torch.zeros(4, 32, dtype=torch.uint8), torch.zeros(4)
+    with pytest.warns(RuntimeWarning, match="native call path"):
+        f = N.fast()
+    assert f is N.fast()
+    assert f.grouped_forward(x, w, ws, None, 4, 8, None, -1) is None and f.tokenwise_quantize(x, 8) is None
+    with pytest.raises(RuntimeError, match="CUDA required"):
+        N.grouped_forward(x, w, ws, None, 4, 8)
+
+
+@pytest.mark.gpu
+def test_results_without_the_extension(monkeypatch, tmp_path):
+    packed, scales = _layer(48, 128, 4)
+    rows = torch.randn(4, 128, device=DEV, dtype=torch.bfloat16)
+    want = N.grouped_forward(rows, packed, scales, None, 4, 8)
+    monkeypatch.setattr(N, "FAST_PATH", tmp_path / "missing.so")
+    monkeypatch.setattr(N, "_FAST", None)
+    with pytest.warns(RuntimeWarning, match="native call path"):
+        assert torch.equal(N.grouped_forward(rows, packed, scales, None, 4, 8), want)
+    codes, s = N.quantize_groups(rows, 8)
+    assert torch.equal(N.grouped_linear(codes, s, packed, scales, None, rows, 4, 8), want)
+
+
+def test_the_extension_is_built_again_for_another_torch(monkeypatch, tmp_path):
+    from actune_amd import build as B
+    lib = tmp_path / B.BINDING_LIB.name
+    lib.write_bytes(b"")
+    monkeypatch.setattr(B, "BINDING_LIB", lib)
+    monkeypatch.setattr(B, "BINDING_STAMP", tmp_path / "stamp")
+    assert B._binding_stale()  # of an unknown torch
+    B.BINDING_STAMP.write_text(B._binding_target())
+    assert not B._binding_stale()
+    B.BINDING_STAMP.write_text(B._binding_target().replace(torch.__version__, "1.0.0"))
+    assert B._binding_stale()
