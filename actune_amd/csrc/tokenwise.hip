@@ -26,7 +26,9 @@
 //
 // MFMA operands (v_mfma_i32_16x16x64_i8): output channels are the A operand,
 // tokens the B operand, so that a lane's four results are consecutive
-// channels of one token; lane l holds row l % 16 and the 16 k-slots of
+// channels of one token, one store; the small-M kernel also has the other
+// order (a lane's results are four tokens of one channel), for the calls that
+// launch_gemm_t sends there. Lane l holds row l % 16 and the 16 k-slots of
 // group kb = l / 16. The k index behind each slot only has to be the same
 // for both operands, so each weight layout uses the slot order its bytes
 // give cheapest:
@@ -165,39 +167,99 @@ __device__ __forceinline__ TwArgs for_target(const TwArgs& in, int i) {
   return a;
 }
 
-// Scales and biases of C consecutive columns from n (columns past N: zeros).
+// y for output (m, n) from the true int32 accumulator, in the family's
+// fixed fp32 sequence, stored in out_dt.
+template <int EPI>
+__device__ __forceinline__ void store_result(const TwArgs& a, int m, int n, int32_t acc) {
+  const float x = (float)acc;
+  const float as = a.as[m], ws = a.ws[n] * a.ws_mul;
+  float y;
+  if constexpr (EPI == ACTUNE_TW_EPI_A8) {
+    const float t = x * as;
+    y = a.bias ? __builtin_fmaf(t, ws, load_bias(a.bias, a.bias_dt, n)) : t * ws;
+  } else {
+    const float q = as * ws;
+    y = a.bias ? __builtin_fmaf(x, q, load_bias(a.bias, a.bias_dt, n)) : x * q;
+  }
+  const size_t o = (size_t)m * a.N + n;
+  if (a.out_dt == kBF16) store_out<kBF16>(a.out, o, y);
+  else if (a.out_dt == kF16) store_out<kF16>(a.out, o, y);
+  else store_out<kF32>(a.out, o, y);
+}
+
+// Scales and biases of C consecutive columns. fetch_cols only issues the
+// loads (bits as they are, 16-bit biases in the low half), so that they and
+// whatever the caller loads next are in flight together; finish_cols converts
+// them. (Behind a test of its column and scaled or converted on the spot, each
+// load waits for a round trip of its own.)
+template <int C>
+struct TwRaw {
+  uint32_t ws[C], bias[C];
+};
 template <int C>
 struct TwCols {
   float ws[C], bias[C];
 };
 
-template <int DT, int C, int NT>
-__device__ __forceinline__ void load_bias_cols(const TwArgs& a, int n, TwCols<C> (&c)[NT]) {
+// C dwords of a row of N at columns n .. n + C - 1 (past N: zeros): one load
+// where the row and its base keep them aligned, else one per column
+template <int C>
+__device__ __forceinline__ void fetch_dwords(Rsrc rs, int n, int N, bool vec, uint32_t (&v)[C]) {
+  if constexpr (C == 4) {
+    if (vec) {
+      const v4u q = __builtin_amdgcn_raw_buffer_load_b128(rs, n < N ? (uint32_t)n * 4u : kOff, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = q[r];
+      return;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < C; ++r)
+    v[r] = __builtin_amdgcn_raw_buffer_load_b32(rs, n + r < N ? (uint32_t)(n + r) * 4u : kOff, 0, 0);
+}
+
+// column groups n, n + 16, ... n + 16 (NT - 1)
+template <int C, int NT>
+__device__ __forceinline__ void fetch_cols(const TwArgs& a, int n, TwRaw<C> (&c)[NT]) {
+  const int N = a.N;
+  const Rsrc wr = make_rsrc(a.ws, (uint32_t)N * 4u);
+  const bool wvec = N % 4 == 0 && (uintptr_t)a.ws % 16 == 0;
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) fetch_dwords<C>(wr, n + 16 * nt, N, wvec, c[nt].ws);
+  if (!a.bias) return;
+  if (a.bias_dt == kF32) {
+    const Rsrc br = make_rsrc(a.bias, (uint32_t)N * 4u);
+    const bool bvec = N % 4 == 0 && (uintptr_t)a.bias % 16 == 0;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) fetch_dwords<C>(br, n + 16 * nt, N, bvec, c[nt].bias);
+  } else {
+    const Rsrc br = make_rsrc(a.bias, (uint32_t)N * 2u);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int r = 0; r < C; ++r) {
+        const int at = n + 16 * nt + r;
+        c[nt].bias[r] = __builtin_amdgcn_raw_buffer_load_b16(br, at < N ? (uint32_t)at * 2u : kOff, 0, 0);
+      }
+  }
+}
+
+template <int C, int NT>
+__device__ __forceinline__ void finish_cols(const TwArgs& a, const TwRaw<C> (&raw)[NT], TwCols<C> (&c)[NT]) {
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int r = 0; r < C; ++r) {
-      const int at = n + 16 * nt + r;
-      c[nt].bias[r] = at < a.N ? load_as_f32<DT>(a.bias, at) : 0.f;
+      c[nt].ws[r] = __uint_as_float(raw[nt].ws[r]) * a.ws_mul;
+      c[nt].bias[r] = a.bias ? bias_from_bits(raw[nt].bias[r], a.bias_dt) : 0.f;
     }
 }
 
-// column groups n, n + 16, ... n + 16 (NT - 1): every load is issued before
-// the first is used
-template <int C, int NT>
-__device__ __forceinline__ void load_cols(const TwArgs& a, int n, TwCols<C> (&c)[NT]) {
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int r = 0; r < C; ++r) {
-      const int at = n + 16 * nt + r;
-      c[nt].ws[r] = (at < a.N ? a.ws[at] : 0.f) * a.ws_mul;
-      c[nt].bias[r] = 0.f;
-    }
-  if (!a.bias) return;
-  if (a.bias_dt == kBF16) load_bias_cols<kBF16>(a, n, c);
-  else if (a.bias_dt == kF16) load_bias_cols<kF16>(a, n, c);
-  else load_bias_cols<kF32>(a, n, c);
+// f32_to_bf16 without a branch on NaN: a lane converts up to 96 results
+__device__ __forceinline__ uint32_t bf16_bits(float f) {
+  const uint32_t u = __float_as_uint(f);
+  const uint32_t rounded = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16, nan = (u >> 16) | 0x40u;
+  return f != f ? nan : rounded;
 }
 
 // y of C columns of row m from the true int32 accumulators, in the family's
@@ -226,7 +288,7 @@ __device__ __forceinline__ void store_cols(const TwArgs& a, int m, int n, float 
       } else {
         uint32_t h[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) h[r] = DT == kBF16 ? f32_to_bf16(y[r]) : f32_to_f16(y[r]);
+        for (int r = 0; r < 4; ++r) h[r] = DT == kBF16 ? bf16_bits(y[r]) : f32_to_f16(y[r]);
         *reinterpret_cast<v2u*>((uint16_t*)a.out + o) = v2u{h[0] | h[1] << 16, h[2] | h[3] << 16};
       }
       return;
@@ -273,10 +335,12 @@ __device__ __forceinline__ void finish_tile(const TwArgs& args, const v4i (&acc)
     return;
   }
   float as[MT];
+  TwRaw<4> raw[NT];
   TwCols<4> cols[NT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) as[mt] = row + mt * 16 < M ? args.as[row + mt * 16] : 0.f;
-  load_cols(args, col, cols);
+  for (int mt = 0; mt < MT; ++mt) as[mt] = args.as[min(row + mt * 16, M - 1)];  // (rows past M are not stored)
+  fetch_cols(args, col, raw);
+  finish_cols(args, raw, cols);
   const bool wide = wide_rows(args.out, args.out_dt, N);
   auto emit = [&](auto dt) {
 #pragma unroll
@@ -294,6 +358,40 @@ __device__ __forceinline__ void finish_tile(const TwArgs& args, const v4i (&acc)
   if (args.out_dt == kBF16) emit(std::integral_constant<int, kBF16>{});
   else if (args.out_dt == kF16) emit(std::integral_constant<int, kF16>{});
   else emit(std::integral_constant<int, kF32>{});
+}
+
+// The same with the operands in the other order (lane: rows row_base + 16 mt +
+// 0..3, column col_base + 16 nt).
+template <int WL, int AL, int EPI, int MT, int NT>
+__device__ __forceinline__ void finish_rows(const TwArgs& args, const v4i (&acc)[MT][NT], int row_base,
+                                            int col_base, int z) {
+  constexpr int SHIFT = WTraits<WL>::TW + (AL == ACTUNE_TW_ACT_A4 ? 4 : 0);
+  const int M = args.M, N = args.N;
+  if (args.splits > 1) {
+    int32_t* part = args.partial + (size_t)z * M * N;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = row_base + mt * 16 + i, n = col_base + nt * 16;
+          if (m < M && n < N) part[(size_t)m * N + n] = acc[mt][nt][i];
+        }
+    return;
+  }
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int n = col_base + nt * 16;
+    if (n >= N) continue;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = row_base + mt * 16 + i;
+        if (m < M) store_result<EPI>(args, m, n, acc[mt][nt][i] >> SHIFT);
+      }
+  }
 }
 
 // Bytes of 16 q4 + r4 as int8, wrapped to 8 bits (decode_w4a8_triton.py:61-66
@@ -347,7 +445,9 @@ constexpr int align_of_stride(int s) { return s % 16 == 0 ? 16 : (s % 8 == 0 ? 8
 // clamped to [-128, 127] exactly as tw_quantize_kernel does, and stages the
 // codes as the activation tile. The first workgroup writes the scales to
 // args.as (the integer reduce reads them).
-template <int WL, int AL, int EPI, int WM, int MT, int NT, int NB, int XDT = -1, int XR = 1>
+//
+// ROWS: the operand order (launch_gemm_t chooses).
+template <int WL, int AL, int EPI, int WM, int MT, int NT, int NB, bool ROWS, int XDT = -1, int XR = 1>
 __global__ __launch_bounds__(kThreads) void tw_gemm(const TwArgs args_in) {
   const int target = (int)blockIdx.z / args_in.splits;
   const TwArgs args = for_target(args_in, target);
@@ -529,7 +629,8 @@ __global__ __launch_bounds__(kThreads) void tw_gemm(const TwArgs args_in) {
           else if constexpr (WL == ACTUNE_TW_ROWS_S2) reorder_slot<8, 2>(af);
         }
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = mfma16x16x64(bf[nt], af, acc[mt][nt]);
+        for (int nt = 0; nt < NT; ++nt)
+          acc[mt][nt] = ROWS ? mfma16x16x64(af, bf[nt], acc[mt][nt]) : mfma16x16x64(bf[nt], af, acc[mt][nt]);
       }
     }
   };
@@ -727,7 +828,8 @@ __global__ __launch_bounds__(kThreads) void tw_gemm(const TwArgs args_in) {
 #pragma unroll
   for (int i = 0; i < NB; ++i) compute(i);
 
-  finish_tile<WL, AL, EPI, MT, NT>(fin, acc, m0 + wm * 16 * MT + r16, n0 + wn * 16 * NT + 4 * kb, z);
+  if constexpr (ROWS) finish_rows<WL, AL, EPI, MT, NT>(fin, acc, m0 + wm * 16 * MT + 4 * kb, n0 + wn * 16 * NT + r16, z);
+  else finish_tile<WL, AL, EPI, MT, NT>(fin, acc, m0 + wm * 16 * MT + r16, n0 + wn * 16 * NT + 4 * kb, z);
 }
 
 // ------------------------------------------------------------ LDS-DMA ring
@@ -1086,11 +1188,11 @@ __global__ __launch_bounds__(kThreads) void tw_reduce(const TwArgs args_in, int 
   const Rsrc pr = make_rsrc(args.partial, (uint32_t)S * total * 4u);
   const bool quads = CPT == 4 && (N & 3) == 0;
   const bool wide = CPT == 4 && wide_rows(args.out, args.out_dt, N);
-  TwCols<CPT> cols[1];
-  load_cols(args, n0, cols);
+  TwRaw<CPT> raw[1];
+  if constexpr (CPT == 4) fetch_cols(args, n0, raw);
   for (int m = (int)blockIdx.y; m < M; m += (int)gridDim.y) {
     const uint32_t base = (uint32_t)m * (uint32_t)N + (uint32_t)n0;
-    const float as = args.as[m];
+    const float as = CPT == 4 ? args.as[m] : 0.f;
     int32_t sum[CPT] = {};
     for (int s0 = 0; s0 < S; s0 += NS) {
       int32_t v[NS][CPT];
@@ -1117,6 +1219,12 @@ __global__ __launch_bounds__(kThreads) void tw_reduce(const TwArgs args_in, int 
     }
 #pragma unroll
     for (int r = 0; r < CPT; ++r) sum[r] >>= shift;
+    if constexpr (CPT == 1) {
+      store_result<EPI>(args, m, n0, sum[0]);
+      continue;
+    }
+    TwCols<CPT> cols[1];
+    finish_cols(args, raw, cols);
     if (args.out_dt == kBF16) store_cols<EPI, kBF16>(args, m, n0, as, cols[0], sum, wide);
     else if (args.out_dt == kF16) store_cols<EPI, kF16>(args, m, n0, as, cols[0], sum, wide);
     else store_cols<EPI, kF32>(args, m, n0, as, cols[0], sum, wide);
@@ -1306,12 +1414,22 @@ void launch_reduce(const TwArgs& a, int shift, hipStream_t st) {
   else launch_reduce_c<EPI, 1>(a, shift, st);
 }
 
+// The operand order: with the channels first, finish_tile gives the row or two
+// of the smallest calls to 4 or 8 of a wave's 64 lanes, which walk eight
+// results each; with the tokens first 16 lanes take two or four (unsplit, one
+// row: 8192 x 256 W2A8 5.2 against 4.3 us, 4096 x 256 W8A8 4.1 / 3.7; from
+// three rows on the other way round: 4096 x 256 W8A4 at three 4.25 / 4.76, at
+// 16 W8A8 4.0 / 5.1). Of split calls, which store raw sums, W8 is 1-2% faster
+// channels first, W2 2-4% slower, the others within 1%.
 template <int WL, int AL, int EPI, int WM, int MT, int NT, int NB, int XDT = -1, int XR = 1>
 void launch_gemm_t(const TwArgs& a, hipStream_t st) {
   constexpr int TM = 16 * MT * WM, TN = 16 * NT * (4 / WM);
   const dim3 grid((unsigned)((a.N + TN - 1) / TN), (unsigned)((a.M + TM - 1) / TM),
                   (unsigned)(a.splits * a.targets));
-  tw_gemm<WL, AL, EPI, WM, MT, NT, NB, XDT, XR><<<grid, kThreads, 0, st>>>(a);
+  if (a.splits > 1 ? WL != ACTUNE_TW_KMAJOR_W8 : a.M <= 2)
+    tw_gemm<WL, AL, EPI, WM, MT, NT, NB, true, XDT, XR><<<grid, kThreads, 0, st>>>(a);
+  else
+    tw_gemm<WL, AL, EPI, WM, MT, NT, NB, false, XDT, XR><<<grid, kThreads, 0, st>>>(a);
   if (a.splits > 1) launch_reduce<EPI>(a, WTraits<WL>::TW + (AL == ACTUNE_TW_ACT_A4 ? 4 : 0), st);
 }
 

@@ -44,3 +44,40 @@ def test_misaligned_outputs(dtype, m, n, k):
         assert shift == 0 or buf[0] == 7.0
     want = (codes.double() @ w.double()).float() * scales.view(-1, 1) * ws
     assert torch.equal(outs[0], want.to(dtype)) and torch.equal(outs[1], outs[0])
+
+
+# scales and biases at every alignment that the call takes: one row without and with a K split, the ring without and with
+# one (its reduce with one and with four columns a thread); 130 rows of weights: no whole groups of four columns
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1, 144, 256), (3, 4096, 512), (1, 1024, 4096), (40, 130, 256), (300, 1024, 4096),
+                                   (600, 8192, 256)])
+@pytest.mark.parametrize("bias_dtype", [torch.float32, torch.bfloat16, torch.float16, None])
+@pytest.mark.parametrize("layout", [N.TW_KMAJOR_W8, N.TW_ROWS_S4])
+def test_scales_and_biases_at_any_alignment(layout, bias_dtype, m, n, k):
+    if layout == N.TW_KMAJOR_W8:
+        n = -(-n // 16) * 16
+    torch.manual_seed(m + n)
+    act, size = (N.TW_ACT_A8, k * n) if layout == N.TW_KMAJOR_W8 else (N.TW_ACT_A4, k // 2 * n)
+    w = torch.randint(-128, 128, (size,), device="cuda:0", dtype=torch.int8)
+    codes, scales = N.tokenwise_quantize(torch.randn(m, k, device="cuda:0"), 8 if act == N.TW_ACT_A8 else 4)
+    work = torch.empty(N.tokenwise_workspace_bytes(m, n, k, layout, act), device="cuda:0", dtype=torch.uint8)
+    outs = []
+    for shift in range(3):
+        gen = torch.Generator(device="cuda:0").manual_seed(9)
+        values, biases = torch.rand(n, device="cuda:0", generator=gen), torch.randn(n, device="cuda:0", generator=gen)
+        ws = torch.full((n + 4,), 1e30, device="cuda:0")
+        ws[shift:shift + n] = values
+        bias = None
+        if bias_dtype is not None:
+            bias = torch.full((n + 4,), 1e4, device="cuda:0", dtype=bias_dtype)
+            bias[shift:shift + n] = biases.to(bias_dtype)
+        out = torch.empty(m, n, device="cuda:0")
+        N.tokenwise_linear(codes, act, scales, w, layout, ws[shift:shift + n], None if bias is None else bias[shift:shift + n],
+                           n, k, N.TW_EPI_A8, out, work)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    if layout == N.TW_KMAJOR_W8:
+        acc = (codes.double() @ w.view(k, n).double()).float() * scales.view(-1, 1)
+        want = acc * values if bias is None else (acc.double() * values.double() + biases.to(bias_dtype).double()).float()
+        # one fma; the reference's sum in double rounds once more
+        torch.testing.assert_close(outs[0], want, rtol=0 if bias is None else 2 ** -22, atol=0)
