@@ -148,6 +148,7 @@ struct TwArgs {
   const uint8_t* r;     // KMAJOR_W4R4: residual codes (nullptr: r4 = 0)
   float ws_mul;         // 1, or 1/16 for the nested 16 q4 + r4 codes (exact)
   int M, N, K, bias_dt, out_dt, splits, steps;
+  uint32_t div_band, div_last;  // ring_tile's reciprocals (0: tiles in row order)
   int targets;          // T: grid z = S x T (GEMM), T (reduce)
   TwTarget t[ACTUNE_MAX_TARGETS];
 };
@@ -869,18 +870,24 @@ __device__ __forceinline__ constexpr int lds_pos(int r, int b) {
 
 // The tile (column, row) of a ring workgroup. Workgroups go to the 8 XCDs in
 // turn, each with its own L2: an XCD takes a contiguous eighth of the tiles,
-// counted down columns of 8 tile rows, so that the workgroups it holds at a
-// time form a near-square block and share its weight and activation tiles
-// (1500 x 11008 x 4096 W8A8: 147 us in row order, 138 in this one).
-__device__ __forceinline__ int2 ring_tile() {
-  constexpr int kXcds = 8, kRows = 8;
-  const int cols = (int)gridDim.x, rows = (int)gridDim.y, total = cols * rows;
-  const int id = (int)blockIdx.x + cols * (int)blockIdx.y;
-  const int xcd = id % kXcds;
-  const int t = xcd * (total / kXcds) + min(xcd, total % kXcds) + id / kXcds;
-  const int first = t / (kRows * cols) * kRows, high = min(kRows, rows - first);
-  const int in = t - first * cols;
-  return make_int2(in / high, first + in % high);
+// counted down columns of kBandRows tile rows, so that the workgroups it holds
+// at a time form a near-square block and share its weight and activation tiles
+// (1500 x 11008 x 4096 W8A8: 147 us in row order, 138 in this one; 200 x 1696
+// x 8704 W8A8 24.1 and 17.0). The host passes reciprocals in place of the two
+// divisions (div_by), or zero where the row order is taken (ring_order).
+constexpr int kXcds = 8, kBandRows = 8;
+
+template <int TM, int TN>
+__device__ __forceinline__ int2 ring_tile(const TwArgs& args) {
+  const int2 plain = make_int2((int)blockIdx.x, (int)blockIdx.y);
+  if (!args.div_band) return plain;
+  const uint32_t cols = (uint32_t)(args.N + TN - 1) / TN, rows = (uint32_t)(args.M + TM - 1) / TM, total = cols * rows;
+  const uint32_t id = blockIdx.x + cols * blockIdx.y, xcd = id % kXcds;
+  const uint32_t t = xcd * (total / kXcds) + min(xcd, total % kXcds) + id / kXcds;
+  const uint32_t first = __umulhi(t, args.div_band) * kBandRows, in = t - first * cols;
+  const uint32_t high = min((uint32_t)kBandRows, rows - first);
+  const uint32_t col = high == kBandRows ? in / kBandRows : high == 1 ? in : __umulhi(in, args.div_last);
+  return make_int2((int)col, (int)(first + in - col * high));
 }
 
 // Large-M tokenwise GEMM: the tile geometry of tw_gemm, with the K-steps
@@ -911,7 +918,7 @@ __global__ __launch_bounds__(kThreads) void tw_gemm_ring(const TwArgs args_in) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
-  const int2 tile = ring_tile();
+  const int2 tile = ring_tile<TM, TN>(args_in);
   const int n0 = tile.x * TN, m0 = tile.y * TM;
   const int z = (int)blockIdx.z % args.splits;
   const int g0 = (int)((long)z * args.steps / args.splits), g1 = (int)((long)(z + 1) * args.steps / args.splits);
@@ -1442,6 +1449,16 @@ constexpr size_t ring_lds_bytes() {
   return (size_t)D * KS * SUB + ((SUB / 1024) % 4 ? 4096 : 0);
 }
 
+// n / d == umulhi(n, div_by(d)) for every n with n * d < 2^32 (d > 1)
+uint32_t div_by(uint32_t d) { return (uint32_t)((1ull << 32) / d + 1); }
+
+// Whether the ring's tiles go to the XCDs in blocks (ring_tile): not up to
+// 1024 columns, whose eight tile columns the row order already gives an XCD
+// each (65 x 1024 x 2048 W4A8 7.6 us, 7.9 in blocks) - unless they are W8
+// columns that end inside a 128-byte line, which neighbours in one L2 read once
+// (300 x 608 x 10752: 17.0 us, 14.1 in blocks).
+bool ring_order(int wl, int N) { return N > 1024 || (wl == ACTUNE_TW_KMAJOR_W8 && N % 128 != 0); }
+
 template <int WL, int AL, int EPI, int WM, int MT, int NT, int KS, int D>
 void launch_ring_t(const TwArgs& a, hipStream_t st) {
   constexpr int TM = 16 * MT * WM, TN = 16 * NT * (4 / WM);
@@ -1450,7 +1467,14 @@ void launch_ring_t(const TwArgs& a, hipStream_t st) {
   if constexpr (lds > 64 * 1024) allow_dynamic_lds<tw_gemm_ring<WL, AL, EPI, WM, MT, NT, KS, D>>();
   const dim3 grid((unsigned)((a.N + TN - 1) / TN), (unsigned)((a.M + TM - 1) / TM),
                   (unsigned)(a.splits * a.targets));
-  tw_gemm_ring<WL, AL, EPI, WM, MT, NT, KS, D><<<grid, kThreads, lds, st>>>(a);
+  TwArgs b = a;
+  const uint64_t band = (uint64_t)kBandRows * grid.x;
+  if (ring_order(WL, a.N) && (uint64_t)grid.x * grid.y * band < 1ull << 32) {
+    const uint32_t last = grid.y % kBandRows;
+    b.div_band = div_by((uint32_t)band);
+    b.div_last = last > 1 ? div_by(last) : 0;
+  }
+  tw_gemm_ring<WL, AL, EPI, WM, MT, NT, KS, D><<<grid, kThreads, lds, st>>>(b);
   if (a.splits > 1) launch_reduce<EPI>(a, WTraits<WL>::TW + (AL == ACTUNE_TW_ACT_A4 ? 4 : 0), st);
 }
 

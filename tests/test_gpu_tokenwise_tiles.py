@@ -81,3 +81,16 @@ def test_scales_and_biases_at_any_alignment(layout, bias_dtype, m, n, k):
         want = acc * values if bias is None else (acc.double() * values.double() + biases.to(bias_dtype).double()).float()
         # one fma; the reference's sum in double rounds once more
         torch.testing.assert_close(outs[0], want, rtol=0 if bias is None else 2 ** -22, atol=0)
+
+
+# the tile order of the ring: one band of tile rows or several, a last band of one, two or all eight, tiles that do not
+# divide over the XCDs, up to 1024 columns (row order, but for W8 columns that end inside a line) and past them
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n", [(33, 1104), (190, 2064), (512, 1168), (513, 1040), (640, 1552), (1090, 1040), (600, 608),
+                                 (600, 1024)])
+@pytest.mark.parametrize("layer", [T.W8A8TritonLinear, T.W4A8TritonLinear, T.W2A4NativeLinear])
+def test_tile_order_reaches_every_tile(layer, m, n):
+    torch.manual_seed(m + n)
+    lay = layer(torch.nn.Linear(256, n, device="cuda:0", dtype=torch.bfloat16))
+    x = torch.randn(m, 256, device="cuda:0", dtype=torch.bfloat16)
+    assert torch.equal(lay(x), torch.cat([lay(part) for part in x.split(32)]))
