@@ -1335,11 +1335,14 @@ int64_t tiles_of(int64_t M, int64_t N, const Geometry& g) {
 // Up to 256 tiles, one per CU: 4 slots of two K-steps, so that one workgroup
 // alone keeps enough bytes in flight (512 x 4096 x 4096 W8A8, quantizer
 // included: 18.8 us, 26.4 us with 3 slots of one), on 64 x 64 tiles for the
-// row-major layouts. Up to 511, two per CU: what leaves LDS for two, 3 slots
-// of two K-steps for W8 and the row-major layouts (300 x 11008 x 4096 W8A8:
-// 26.8 us, 33.9 with 4 slots, 32.5 with one K-step), 4 of two for the nibble
-// pairs (26.7; 30.7 with 3 of one), 3 of one for the quarters, whose
-// activation tile is twice as wide (25.1; 34.8).
+// row-major layouts, up to 384 tiles there (three of 64 x 64 per CU: 705 x
+// 2768 x 4096 W4A4, 264 tiles, 21.7 us, 26.0 with 64 x 128; from 385 on the
+// fourth round costs more, 2162 x 1824 x 11008 W2A4 79.4 against 62.8). Up to
+// 511, two per CU: what leaves LDS for two, 3 slots of two K-steps for W8 and
+// the row-major layouts (300 x 11008 x 4096 W8A8: 26.8 us, 33.9 with 4 slots,
+// 32.5 with one K-step), 4 of two for the nibble pairs (26.7; 30.7 with 3 of
+// one), 3 of one for the quarters, whose activation tile is twice as wide
+// (25.1; 34.8).
 //
 // From 512 on the grid runs in rounds of one tile per CU, with two or three
 // in flight, and a tile of 96, 128 or (W8) 192 rows reads fewer weight bytes
@@ -1356,7 +1359,7 @@ Geometry pick_geometry(int64_t M, int64_t N, int wl) {
   const int ks = km ? 1 : 2;
   const Geometry base{2, 2, 4, 0, ks, 3}, deep{2, 2, 4, 0, 2, 4};
   const int64_t tiles = tiles_of(M, N, base);
-  if (tiles <= 256) return km ? deep : Geometry{2, 2, 2, 0, 2, 4};
+  if (tiles <= (km ? 256 : 384)) return km ? deep : Geometry{2, 2, 2, 0, 2, 4};
   if (tiles < 512) {
     if (wl == ACTUNE_TW_KMAJOR_W4) return deep;
     return wl == ACTUNE_TW_KMAJOR_W2 ? base : Geometry{2, 2, 4, 0, 2, 3};

@@ -94,3 +94,14 @@ def test_tile_order_reaches_every_tile(layer, m, n):
     lay = layer(torch.nn.Linear(256, n, device="cuda:0", dtype=torch.bfloat16))
     x = torch.randn(m, 256, device="cuda:0", dtype=torch.bfloat16)
     assert torch.equal(lay(x), torch.cat([lay(part) for part in x.split(32)]))
+
+
+# row-major layouts at 257, 384 (64 x 64 tiles) and 385 tiles of 64 x 128
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n", [(16448, 70), (1022, 3010), (4900, 530)])
+@pytest.mark.parametrize("layer", [T.W4A4NativeLinear, T.W2A4NativeLinear])
+def test_row_major_tiles(layer, m, n):
+    torch.manual_seed(m + n)
+    lay = layer(torch.nn.Linear(128, n, device="cuda:0", dtype=torch.bfloat16))
+    x = torch.randn(m, 128, device="cuda:0", dtype=torch.bfloat16)
+    assert torch.equal(lay(x), torch.cat([lay(part) for part in x.split(32)]))
