@@ -89,6 +89,7 @@ int check_target(const uint8_t* w, const float* ws, const void* out, int64_t N, 
 }
 
 int packed_default(int64_t M, int64_t N, int64_t K, int W, int A);
+int forward_default(int64_t M, int64_t N, int64_t K, int W, int A);
 
 // Whether a decode-config call quantizes x inside the GEMM. Every workgroup
 // quantizes the whole activation, so the in-launch work grows as workgroups
@@ -137,14 +138,15 @@ bool selectable(int64_t M, int64_t N, int64_t K, int W, int A) {
 }
 
 // ACTUNE_CONFIG_AUTO: calls that hand over x (and may fuse the quantizer) use
-// actune_default_config; calls on packed activations use packed_default (the
-// same choice without the in-launch quantization). Arguments no call takes
+// forward_default; calls on packed activations use packed_default (the same
+// choice without the in-launch quantization), above 16 tokens plan_codes in
+// its place. Arguments no call takes
 // resolve to the first prefill config, valid at every M, so that the call's
 // own checks name what is wrong.
 int resolve(int config, int64_t M, int64_t N, int64_t K, int W, int A, bool has_x) {
   if (config != ACTUNE_CONFIG_AUTO) return config;
   if (!selectable(M, N, K, W, A)) return kPrefillFirst;
-  return has_x ? actune_default_config(M, N, K, W, A) : packed_default(M, N, K, W, A);
+  return has_x ? forward_default(M, N, K, W, A) : packed_default(M, N, K, W, A);
 }
 
 // Fill the problem table of a launch; returns the number of 16-row tiles.
@@ -242,10 +244,10 @@ bool decode_waves_useful(int64_t K, int nw) {
   const int64_t q = (K / kGroup + 3) / 4;
   return nw <= 4 || nw <= q;
 }
-}  // namespace
 
-int actune_default_config(int64_t M, int64_t N, int64_t K, int W, int A) {
-  if (!selectable(M, N, K, W, A)) return ACTUNE_CONFIG_AUTO;
+// The config of a forward call that takes x, where it runs as one launch on x
+// or, up to 16 tokens, on the quantizer's codes.
+int forward_default(int64_t M, int64_t N, int64_t K, int W, int A) {
   // Decode (M <= 64, measured on MI355X at Llama/Gemma shapes): the decode
   // kernel beats the small-M and streaming kernels wherever a wave's K-range
   // fits its load ring. Calls that hand over bf16 x first try to quantize it
@@ -314,7 +316,6 @@ int actune_default_config(int64_t M, int64_t N, int64_t K, int W, int A) {
   return packed_default(M, N, K, W, A);
 }
 
-namespace {
 // The decode config for a call on packed codes, or -1 where no wave count
 // fits (measured on MI355X, W2/W4/W8 x A4/A8, M = 1..64): M <= 4 and narrow
 // N, the fewest waves that still give every SIMD a wave; wide N (more than
@@ -444,27 +445,26 @@ int prefill_choice(int64_t M, int64_t N, int64_t K, int W, float* us) {
   return kPrefillCostConfig[best];
 }
 
-// Runs the problems of g (one width, M > 16) on codes with the kernel of the
-// least estimated time.
-void run_planned(int W, int A, const LinearArgs& g, hipStream_t st) {
-  const int64_t M = g.M, K = g.K;
+// The config of a call on codes above 16 tokens under ACTUNE_CONFIG_AUTO, for
+// problems of n[0 .. nprob) rows: one launch over all of them, or kPerProblem:
+// a prefill launch each (prefill_choice).
+constexpr int kPerProblem = -1;
+
+int plan_codes(int64_t M, int64_t K, const int64_t* n, int nprob, int W, int A) {
   int64_t n_total = 0;
-  for (int q = 0; q < g.nprob; ++q) n_total += g.prob[q].N;
+  for (int q = 0; q < nprob; ++q) n_total += n[q];
   const int single = packed_default(M, n_total, K, W, A);
-  if (M > kDecodeAutoMax && single >= kDecodeFirst) {  // narrow problems keep the decode kernel
-    run_gemm(W, A, single, kModePacked, g, st);
-    return;
-  }
+  if (M > kDecodeAutoMax && single >= kDecodeFirst) return single;  // narrow problems keep the decode kernel
   float best = 0.f, us = 0.f;
-  int config = -1;  // one launch over every problem; -1: prefill, problem by problem
-  for (int q = 0; q < g.nprob; ++q) {
-    prefill_choice(M, g.prob[q].N, K, W, &us);
+  int config = kPerProblem;
+  for (int q = 0; q < nprob; ++q) {
+    prefill_choice(M, n[q], K, W, &us);
     best += us;
   }
   for (int i = 0; i < 3; ++i) {
     const TileCost& c = kWideCost[W == 8][i];
     int64_t tiles = 0;
-    for (int q = 0; q < g.nprob; ++q) tiles += tiles_of(c, M, g.prob[q].N);
+    for (int q = 0; q < nprob; ++q) tiles += tiles_of(c, M, n[q]);
     us = launch_cost(c, tiles, K);
     if (us <= best) { best = us; config = kWideFirst + i; }
   }
@@ -474,7 +474,15 @@ void run_planned(int W, int A, const LinearArgs& g, hipStream_t st) {
     us = (float)K / 4096.f * blocks / 1024.f * (W == 8 ? 21.f : fits ? 11.3f : 20.f);
     if (us <= best) config = single;
   }
-  if (config >= 0) {
+  return config;
+}
+
+// Runs the problems of g (one width, M > 16) on codes as plan_codes says.
+void run_planned(int W, int A, const LinearArgs& g, hipStream_t st) {
+  int64_t n[kMaxProblems];
+  for (int q = 0; q < g.nprob; ++q) n[q] = g.prob[q].N;
+  const int config = plan_codes(g.M, g.K, n, g.nprob, W, A);
+  if (config != kPerProblem) {
     run_gemm(W, A, config, kModePacked, g, st);
     return;
   }
@@ -484,7 +492,8 @@ void run_planned(int W, int A, const LinearArgs& g, hipStream_t st) {
     one.prob[0].tile0 = 0;
     one.nprob = 1;
     one.tiles = (g.prob[q].N + 15) / 16;
-    run_gemm(W, A, prefill_choice(M, g.prob[q].N, K, W, &us), kModePacked, one, st);
+    float us;
+    run_gemm(W, A, prefill_choice(g.M, n[q], g.K, W, &us), kModePacked, one, st);
   }
 }
 
@@ -495,6 +504,15 @@ void run_codes(int W, int A, int config, bool auto_config, const LinearArgs& g, 
   else run_gemm(W, A, config, kModePacked, g, st);
 }
 }  // namespace
+
+int actune_default_config(int64_t M, int64_t N, int64_t K, int W, int A) {
+  if (!selectable(M, N, K, W, A)) return ACTUNE_CONFIG_AUTO;
+  const int config = forward_default(M, N, K, W, A);
+  if (M <= kStreamMax || forward_fuses(config, M, N, K, W, kBF16)) return config;
+  const int planned = plan_codes(M, K, &N, 1, W, A);
+  float us;
+  return planned == kPerProblem ? prefill_choice(M, N, K, W, &us) : planned;
+}
 
 int actune_forward_fuses_quantizer(int64_t M, int64_t N, int64_t K, int W, int A, int x_dtype, int config) {
   g_err[0] = 0;

@@ -121,6 +121,12 @@ def run_only(torch, _native, name, W, A, config):
                           config=cfg if cfg >= 0 else _native.default_config(m, spec[0][0], k, W, A))))
 
 
+def kernel_of(config):
+    """The kernel of a group-64 configuration id (include/actune_hip.h)."""
+    first = ((14, "gemm_decode"), (10, "gemm_prefill"), (7, "gemm_stream"), (3, "gemm_wide"), (0, "gemm_smallm"))
+    return next(name for c, name in first if config >= c)
+
+
 def build_stack(torch, m, layers, W, A, seed=0):
     """Per layer and shape: packed weights, scales, input, scratch, output."""
     g = torch.Generator(device="cuda").manual_seed(seed)
@@ -393,7 +399,9 @@ def bench_prefill(torch, _native, steps, warmup):
         out[f"W{W}A{A}"] = row
     best = {pair: max(v["frac"] for v in out[pair].values()) for pair in ("W8A8", "W4A8")}
     out["roofline"] = {"bound": "mfma", "unit": "TOPS", "peak": INT8_PEAK_TOPS,
-                       "kernel": "gemm_prefill (int8 MFMA + per-group fp32 rescale)",
+                       "kernel": " / ".join(sorted({kernel_of(v["config"]) for pair in ("W4A8", "W8A8")
+                                                    for v in out[pair].values()})) +
+                                 " (int8 MFMA + per-group fp32 rescale)",
                        "W4A8_frac_best_shape": best["W4A8"], "W8A8_frac_best_shape": best["W8A8"],
                        "note": "2 VALU per (token, channel, group) against 64 MACs caps int8 MFMA use at 50%"}
     return out

@@ -174,13 +174,13 @@ int actune_grouped_dots_i32(const uint8_t* a, const uint8_t* w, int64_t M, int64
  *            wave's load ring and the dots mode run the small-M kernel with
  *            the same waves)
  * actune_config_valid: 1 if `config` can run a call with M rows.
- * actune_default_config: the config ACTUNE_CONFIG_AUTO resolves to in
- *   actune_grouped_forward(_multi). actune_grouped_linear and
- *   actune_grouped_dots_i32 (packed activations) resolve AUTO to the same
- *   kernels without the in-launch quantization (a decode config where the
- *   decode kernel fits the codes). Above 16 tokens an AUTO call on codes runs
- *   the kernel of the least estimated time instead (bit-identical). For a width or dimension that no call
- *   takes it returns ACTUNE_CONFIG_AUTO (-1); a call with such arguments
+ * actune_default_config: the config an ACTUNE_CONFIG_AUTO call of
+ *   actune_grouped_forward on bf16 x runs. actune_grouped_linear and
+ *   actune_grouped_dots_i32 (packed activations) resolve AUTO without the
+ *   in-launch quantization (a decode config where the decode kernel fits the
+ *   codes); above 16 tokens AUTO calls on codes, sibling calls among them,
+ *   weigh the kernels' estimated times (bit-identical results). For a width
+ *   or dimension that no call takes it returns ACTUNE_CONFIG_AUTO (-1); a call with such arguments
  *   returns ACTUNE_ERR_INVALID naming them, whatever its config.
  */
 int actune_num_configs(void);

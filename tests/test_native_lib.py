@@ -126,11 +126,11 @@ def test_config_table():
     assert _native.default_config(8, 8192, 1024, 2, 4) == 14
     assert _native.default_config(4, 8192, 1024, 4, 4) == 14
     import torch
-    # from 1024 row tiles above 16 tokens: 16 waves for K >= 4096, 4 below
-    assert _native.default_config(32, 22016, 4096, 4, 8) == 16
-    assert _native.default_config(50, 22016, 4096, 8, 8) == 16
-    assert _native.default_config(50, 32768, 2048, 4, 4) == 14
-    assert _native.default_config(24, 16384, 2048, 4, 4) == 14
+    # from 1024 row tiles above 16 tokens the planned kernels are ahead of the decode kernel
+    assert _native.default_config(32, 22016, 4096, 4, 8) == 13
+    assert _native.default_config(50, 22016, 4096, 8, 8) == 4
+    assert _native.default_config(50, 32768, 2048, 4, 4) == 12
+    assert _native.default_config(24, 16384, 2048, 4, 4) == 13
     # W8 at 2-4 tokens takes at most 8 waves; W2 at K >= 4096 takes 16
     assert _native.default_config(2, 1024, 4096, 8, 4) == 15
     assert _native.default_config(4, 1024, 1024, 8, 8) == 14
@@ -165,14 +165,26 @@ def test_config_table():
     assert _native.default_config(128, 1024, 1024, 4, 4) == 14
     assert _native.default_config(256, 512, 4096, 8, 8) == 16
     assert _native.default_config(96, 2048, 16384, 4, 4) == 13  # K above 4096
-    # prefill: 64x32 tiles below two 64x64 tiles per CU, 64x64 below four,
-    # 128x64 from four for W <= 4 (W8 keeps 64x64), the tiled kernel from eight
+    # prefill: 64x32 tiles below two 64x64 tiles per CU, 64x64 or 128x64 or the
+    # wide-tile kernel above
     assert _native.default_config(256, 2048, 2048, 4, 4) == 13
     assert _native.default_config(512, 4096, 4096, 4, 8) == 12
     assert _native.default_config(256, 16384, 2048, 4, 4) == 10
-    assert _native.default_config(512, 11008, 4096, 2, 8) == 10
-    assert _native.default_config(512, 11008, 4096, 8, 8) == 12
+    assert _native.default_config(512, 11008, 4096, 2, 8) == 3
+    assert _native.default_config(512, 11008, 4096, 8, 8) == 5
     assert _native.default_config(2048, 4096, 4096, 4, 8) == 3
+
+
+def test_default_config_is_the_one_an_automatic_call_runs():
+    """Above 16 tokens a call whose quantizer is a launch of its own runs the planned kernel: the choice reported (the
+    tuner's baseline) is that one, not the choice by sizes."""
+    cfg = _native.default_config
+    # the prefill and the wide-tile kernel, where the decode kernel is the choice by sizes
+    assert cfg(40, 11008, 4096, 4, 8) == 13
+    assert cfg(64, 22016, 4096, 8, 8) == 4
+    assert cfg(512, 4096, 4096, 8, 8) == 5
+    # a call that quantizes x in its launch keeps the config that does
+    assert _native.forward_fuses_quantizer(50, 8192, 1024, 4, 4, torch.bfloat16) and cfg(50, 8192, 1024, 4, 4) == 14
 
 
 def _err():
