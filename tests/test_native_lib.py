@@ -178,6 +178,7 @@ def test_config_table():
 def test_default_config_is_the_one_an_automatic_call_runs():
     """Above 16 tokens a call whose quantizer is a launch of its own runs the planned kernel: the choice reported (the
     tuner's baseline) is that one, not the choice by sizes."""
+    import torch
     cfg = _native.default_config
     # the prefill and the wide-tile kernel, where the decode kernel is the choice by sizes
     assert cfg(40, 11008, 4096, 4, 8) == 13
