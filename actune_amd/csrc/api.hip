@@ -394,25 +394,37 @@ int packed_default(int64_t M, int64_t N, int64_t K, int W, int A) {
   return kWideFirst;
 }
 
-// Kernel of a call on codes above 16 tokens under ACTUNE_CONFIG_AUTO: the
-// least estimated time (us) among the decode kernel (up to 64 tokens), the
-// wide-tile kernel over all problems in one launch, and the prefill kernel
-// problem by problem. A launch costs about 6.5 us beyond its walk over K
-// (prologue and epilogue included), the walk K / 4096 times what its
-// TileCost says for the launch's tile count: whole rounds over the 256 CUs where a
-// workgroup fills a CU, measured at one and two workgroups per CU and then
-// proportional to the tiles where several fit.
-// Measured on MI355X (us, K = 4096, hipGraph, rotating weights; W8A8 at N =
+// Kernel of a call on codes above 16 tokens under ACTUNE_CONFIG_AUTO. The
+// choice by sizes (packed_default) keeps the call unless the least estimated
+// time (us) among the wide-tile kernel over all problems in one launch and the
+// prefill kernel problem by problem is lower than its own by kKeep. A launch
+// costs about 6.5 us beyond its walk over K (prologue and epilogue included),
+// the walk K / 4096 times what its TileCost says for the launch's tile count:
+// whole rounds over the 256 CUs where a workgroup fills a CU, measured at one
+// and two workgroups per CU and then proportional to the tiles where several
+// fit. Measured on MI355X (us, K = 4096, hipGraph, rotating weights; W8A8 at N =
 // 4096 / 11008 / 22016, M = 20 .. 2000, and W4A8, W4A4 likewise): W8 128x128
 // tiles 33 per round of 256, 64x128 22, 64x64 18 / 26 up to one / two per CU,
 // prefill 64x32 15.5 up to one per CU; W4 128x64 25 / 38, 64x64 18 / 25,
 // 128x32 16.5 per round, prefill 64x32 11.8, 64x64 17.5 / 24, 128x64 24.5 /
-// 37.5. The decode kernel takes 11.3 (W8: 21) per 1024 blocks of 16 rows x 16
-// tokens, the small-M kernel that stands in for a long K 20 (21). Before
-// this rule 17-64 tokens always took the decode or small-M kernel, and
-// siblings the configuration of their total N: W4A8 11008x4096 at M = 40
-// 27.5 -> 16.2, 4096x11008 at M = 64 44.2 -> 21.6, W8A8 22016x4096 at M = 64
-// 83.8 -> 28.4, 4096x11008 at M = 1024 134.8 -> 87.9.
+// 37.5. W2 takes W4's figures, and every A one figure per kernel; for W2, and
+// W8 with A < 8, the prefill kernel's are up to 15% too high above 512 tiles.
+// W8 prefill takes 0.88 of its figure where K is an odd multiple of 64
+// (measured 10-12% faster there).
+// The estimates scatter: 1500 random sizes (M = 17-2000, N = 256-22016, K =
+// 256-16384, every W and A) lie within 8-12% of them (rms), so kKeep is 7%
+// above 64 tokens and 10% below, against the decode and the small-M kernel,
+// whose estimates scatter most. Sibling problems, where one launch in place of
+// several is most of the gain, take the least estimate (3 x 8192 rows x 8192
+// W8A8 at M = 300: 188 us in one launch, 275 in three); up to 64 tokens, where
+// the decode kernel is one launch as well, it has to be 5% lower.
+// Without kKeep 67 of the 1500 were more than 5% slower than the choice by
+// sizes, up to 32% (W8A4 300 x 17712 x 1600 32.6 -> 40.6 us); with it 20, up
+// to 16%. The whole set takes 0.92 of the time of the
+// choice by sizes, 0.86 with the fastest kernel for every size. The fourth
+// wide-tile shape (64x32, K split) is the fastest of all for 90 of the 1500,
+// few tiles and long K, 6% ahead of the next, but is not weighed here: explicit
+// configs and the tuner run it.
 struct TileCost {
   int bn, bm;           // tile: rows x tokens
   float one, two, per;  // up to 256 and 512 tiles; per tile above (0: `one` per round of 256)
@@ -420,10 +432,11 @@ struct TileCost {
 constexpr TileCost kWideCost[2][3] = {{{128, 64, 25.f, 38.f, 0.0725f}, {64, 64, 18.f, 25.f, 0.0425f}, {128, 32, 16.5f, 0, 0}},
                                       {{128, 128, 33.f, 0, 0}, {64, 64, 18.f, 26.f, 0.0487f}, {64, 128, 22.f, 0, 0}}};
 // prefill configs 10, 12, 13
-constexpr TileCost kPrefillCost[2][3] = {{{128, 64, 24.5f, 37.5f, 0.0785f}, {64, 64, 17.5f, 24.f, 0.041f}, {64, 32, 11.8f, 16.f, 0.036f}},
-                                         {{128, 64, 28.f, 54.f, 0.12f}, {64, 64, 18.5f, 28.f, 0.055f}, {64, 32, 15.5f, 25.f, 0.054f}}};
+constexpr TileCost kPrefillCost[2][3] = {{{128, 64, 24.5f, 37.5f, 0.0785f}, {64, 64, 17.5f, 24.f, 0.041f}, {64, 32, 11.8f, 16.f, 0.032f}},
+                                         {{128, 64, 28.f, 54.f, 0.12f}, {64, 64, 18.5f, 28.f, 0.055f}, {64, 32, 15.5f, 25.f, 0.050f}}};
 constexpr int kPrefillCostConfig[3] = {kPrefillFirst, kPrefillFirst + 2, kPrefillFirst + 3};
 constexpr float kLaunchCost = 6.5f;
+constexpr float kKeep = 0.93f, kKeepDecode = 0.90f, kKeepSiblings = 0.95f;
 
 int64_t tiles_of(const TileCost& c, int64_t M, int64_t N) { return ((N + c.bn - 1) / c.bn) * ((M + c.bm - 1) / c.bm); }
 
@@ -434,15 +447,33 @@ float launch_cost(const TileCost& c, int64_t tiles, int64_t K) {
   return kLaunchCost + (float)K / 4096.f * (t - kLaunchCost);
 }
 
+float prefill_cost(int i, int64_t M, int64_t N, int64_t K, int W) {
+  const TileCost& c = kPrefillCost[W == 8][i];
+  const float t = launch_cost(c, tiles_of(c, M, N), K);
+  return W == 8 && K % 128 ? kLaunchCost + 0.88f * (t - kLaunchCost) : t;
+}
+
 // The prefill config of one problem, and its estimated time.
 int prefill_choice(int64_t M, int64_t N, int64_t K, int W, float* us) {
   int best = 0;
   for (int i = 0; i < 3; ++i) {
-    const TileCost& c = kPrefillCost[W == 8][i];
-    const float t = launch_cost(c, tiles_of(c, M, N), K);
+    const float t = prefill_cost(i, M, N, K, W);
     if (i == 0 || t < *us) { *us = t; best = i; }
   }
   return kPrefillCostConfig[best];
+}
+
+// Estimated time of the decode kernel, and of the small-M kernel that stands in
+// for it where K does not fit its ring (17 to 64 tokens), fitted to the same sizes.
+float decode_cost(int64_t M, int64_t n_total, int64_t K, int W, bool fits) {
+  struct Cost {
+    float launch, k, k_blocks, blocks;  // blocks of 16 rows x 16 tokens, in 1024
+  };
+  static constexpr Cost kDecode[3] = {{4.1f, 1.1f, 6.6f, 0.9f}, {4.2f, 1.2f, 6.4f, 1.2f}, {4.0f, 0.9f, 12.4f, 0.6f}};
+  static constexpr Cost kSmall[3] = {{2.7f, 2.5f, 10.0f, 0.f}, {1.6f, 3.4f, 11.3f, 0.f}, {5.1f, 3.0f, 14.0f, 0.f}};
+  const Cost& c = (fits ? kDecode : kSmall)[W == 2 ? 0 : W == 4 ? 1 : 2];
+  const float blocks = (float)((n_total + 15) / 16 * ((M + 15) / 16)) / 1024.f, k = (float)((K + 255) / 256) / 16.f;
+  return c.launch + k * (c.k + c.k_blocks * blocks) + c.blocks * blocks;
 }
 
 // The config of a call on codes above 16 tokens under ACTUNE_CONFIG_AUTO, for
@@ -454,27 +485,27 @@ int plan_codes(int64_t M, int64_t K, const int64_t* n, int nprob, int W, int A) 
   int64_t n_total = 0;
   for (int q = 0; q < nprob; ++q) n_total += n[q];
   const int single = packed_default(M, n_total, K, W, A);
-  if (M > kDecodeAutoMax && single >= kDecodeFirst) return single;  // narrow problems keep the decode kernel
+  const bool decode = single < kSmallMConfigs || single >= kDecodeFirst;
+  if (M > kDecodeAutoMax && decode) return single;  // narrow problems keep the decode kernel
   float best = 0.f, us = 0.f;
   int config = kPerProblem;
   for (int q = 0; q < nprob; ++q) {
     prefill_choice(M, n[q], K, W, &us);
     best += us;
   }
+  float kept = decode ? decode_cost(M, n_total, K, W, single >= kDecodeFirst) : 0.f;
   for (int i = 0; i < 3; ++i) {
     const TileCost& c = kWideCost[W == 8][i];
     int64_t tiles = 0;
     for (int q = 0; q < nprob; ++q) tiles += tiles_of(c, M, n[q]);
     us = launch_cost(c, tiles, K);
+    if (single == kWideFirst + i) kept = us;
     if (us <= best) { best = us; config = kWideFirst + i; }
+    if (single == kPrefillCostConfig[i])
+      for (int q = 0; q < nprob; ++q) kept += prefill_cost(i, M, n[q], K, W);
   }
-  if (M <= kDecodeAutoMax) {
-    const bool fits = single >= kDecodeFirst;
-    const float blocks = (float)((n_total + 15) / 16 * ((M + 15) / 16));
-    us = (float)K / 4096.f * blocks / 1024.f * (W == 8 ? 21.f : fits ? 11.3f : 20.f);
-    if (us <= best) config = single;
-  }
-  return config;
+  const float keep = nprob > 1 ? (decode ? kKeepSiblings : 1.f) : decode ? kKeepDecode : kKeep;
+  return best < keep * kept ? config : single;
 }
 
 // Runs the problems of g (one width, M > 16) on codes as plan_codes says.

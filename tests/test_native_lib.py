@@ -188,6 +188,17 @@ def test_default_config_is_the_one_an_automatic_call_runs():
     assert _native.forward_fuses_quantizer(50, 8192, 1024, 4, 4, torch.bfloat16) and cfg(50, 8192, 1024, 4, 4) == 14
 
 
+def test_the_plan_keeps_the_choice_by_sizes_unless_clearly_ahead():
+    """Sizes at which the least estimate alone had taken a kernel 15-32% slower than the choice by sizes (measured, us)."""
+    cfg = _native.default_config
+    assert cfg(300, 17712, 1600, 8, 4) == 12  # 32.6; 40.6 in 64x64 wide tiles
+    assert cfg(200, 3120, 704, 8, 8) != 4     # 7.0; 8.3
+    assert cfg(1500, 1024, 11008, 4, 4) == 13  # 49.4; 57.0 in 64x64 tiles
+    assert cfg(1000, 1360, 6656, 4, 4) == 13  # 33.0; 38.2
+    # clear gains stay
+    assert cfg(40, 11008, 4096, 4, 8) != 16 and cfg(64, 22016, 4096, 8, 8) == 4
+
+
 def _err():
     return _native.lib().actune_last_error().decode()
 
