@@ -40,18 +40,20 @@ def test_no_packed_fp32_instructions(device_asm):
 
 
 def test_kernels_use_int8_mfma(device_asm):
-    assert "v_mfma_i32_16x16x64_i8" in device_asm
+    assert "v_mfma_i32_16x16x64_i8" in device_asm and "v_mfma_i32_32x32x32_i8" in device_asm
     assert "buffer_load_dwordx4" in device_asm
 
 
 # ---------------------------------------------------------------- MFMA result hazard
 # A VALU instruction that reads or writes a VGPR written by an int8 MFMA must
 # issue at least MFMA_WAIT wait states after it (every instruction counts one,
-# s_nop N counts N + 1). In straight-line code the compiler never leaves fewer
-# than 8 here; across a branch its wait states have been seen missing (the
-# read then sees the register's old value), so the check follows every
-# control-flow path backwards from each VALU instruction.
-MFMA_WAIT = 8
+# s_nop N counts N + 1): 8 for the four passes of 16x16x64, 4 more for the
+# eight of 32x32x32. In straight-line code the compiler never leaves fewer;
+# across a branch its wait states have been seen missing (the read then sees
+# the register's old value), so the check follows every control-flow path
+# backwards from each VALU instruction.
+MFMA_WAIT = {"v_mfma_i32_16x16x64_i8": 8, "v_mfma_i32_32x32x32_i8": 12}
+MOST_WAIT = max(MFMA_WAIT.values())
 _INS = re.compile(r"^\s+(\S+)\s*(.*?)\s*//\s*([0-9A-Fa-f]+):")
 _FN = re.compile(r"^([0-9a-f]+) <(.+)>:$")
 _TGT = re.compile(r"<(.+)\+0x([0-9a-f]+)>\s*$")
@@ -110,13 +112,15 @@ def _mfma_hazards(ins):
         stack, seen = [(p, 0) for p in preds[k]], set()
         while stack:
             j, ws = stack.pop()
-            if ws >= MFMA_WAIT or (j, ws) in seen:
+            if ws >= MOST_WAIT or (j, ws) in seen:
                 continue
             seen.add((j, ws))
             _a2, op2, args2, _t2 = ins[j]
             if op2.startswith("v_mfma") and _operands(args2)[0] & touched:
-                found.append((hex(a), op, args, ws))
-                break
+                if ws < MFMA_WAIT[op2]:
+                    found.append((hex(a), op, args, ws))
+                    break
+                continue  # the register is this MFMA's: earlier writers do not matter
             step = int(args2.split()[0], 0) + 1 if op2 == "s_nop" else 1
             stack.extend((p, ws + step) for p in preds[j])
     return found
@@ -124,9 +128,19 @@ def _mfma_hazards(ins):
 
 def test_mfma_results_wait_on_every_path(device_asm):
     fns = _functions(device_asm)
-    assert any(any(op.startswith("v_mfma") for _a, op, _x, _t in ins) for ins in fns.values())
+    used = {op for ins in fns.values() for _a, op, _x, _t in ins if op.startswith("v_mfma")}
+    assert used == set(MFMA_WAIT)
     bad = {name: h[:3] for name, ins in fns.items() if (h := _mfma_hazards(ins))}
     assert not bad, f"VALU access to an MFMA result before {MFMA_WAIT} wait states: {bad}"
+
+
+@pytest.mark.parametrize("op", sorted(MFMA_WAIT))
+@pytest.mark.parametrize("short", [1, 0])
+def test_the_wait_check_tells_the_shapes_apart(op, short):
+    """A listing whose VALU read comes one wait state early is found, one at the shape's wait states is not."""
+    lines = [f"{op} v[0:15], v[16:19], v[20:23], 0", f"s_nop {MFMA_WAIT[op] - 1 - short}", "v_mov_b32_e32 v40, v3"]
+    text = "0000000000001000 <kernel>:\n" + "".join(f"\t{x}   // {0x1000 + 8 * i:012X}: 00000000\n" for i, x in enumerate(lines))
+    assert bool(_mfma_hazards(_functions(text)["kernel"])) == bool(short)
 
 
 # ---------------------------------------------------------------- M0 and LDS DMA
