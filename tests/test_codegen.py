@@ -51,9 +51,8 @@ def test_kernels_use_int8_mfma(device_asm):
 # eight of 32x32x32. In straight-line code the compiler never leaves fewer;
 # across a branch its wait states have been seen missing (the read then sees
 # the register's old value), so the check follows every control-flow path
-# backwards from each VALU instruction.
+# from each MFMA.
 MFMA_WAIT = {"v_mfma_i32_16x16x64_i8": 8, "v_mfma_i32_32x32x32_i8": 12}
-MOST_WAIT = max(MFMA_WAIT.values())
 _INS = re.compile(r"^\s+(\S+)\s*(.*?)\s*//\s*([0-9A-Fa-f]+):")
 _FN = re.compile(r"^([0-9a-f]+) <(.+)>:$")
 _TGT = re.compile(r"<(.+)\+0x([0-9a-f]+)>\s*$")
@@ -95,39 +94,47 @@ def _functions(text):
 
 def _mfma_hazards(ins):
     index = {a: k for k, (a, *_rest) in enumerate(ins)}
-    preds = collections.defaultdict(list)
-    for k, (_a, op, _args, t) in enumerate(ins):
-        if k + 1 < len(ins) and op not in _END_FLOW:
-            preds[k + 1].append(k)
-        if t is not None and (op.startswith("s_cbranch") or op == "s_branch") and t in index:
-            preds[index[t]].append(k)
     found = []
-    for k, (a, op, args, _t) in enumerate(ins):
-        if not op.startswith("v_") or op.startswith("v_mfma"):
+    for j, (_a, op, args, _t) in enumerate(ins):
+        if not op.startswith("v_mfma"):
             continue
-        dest, srcs = _operands(args)
-        touched = dest | srcs
-        if not touched:
-            continue
-        stack, seen = [(p, 0) for p in preds[k]], set()
+        # every path from the MFMA, with the wait states so far and its result registers no later MFMA has taken over
+        stack, seen = [(j, 0, frozenset(_operands(args)[0]))], set()
         while stack:
-            j, ws = stack.pop()
-            if ws >= MOST_WAIT or (j, ws) in seen:
-                continue
-            seen.add((j, ws))
-            _a2, op2, args2, _t2 = ins[j]
-            if op2.startswith("v_mfma") and _operands(args2)[0] & touched:
-                if ws < MFMA_WAIT[op2]:
-                    found.append((hex(a), op, args, ws))
-                    break
-                continue  # the register is this MFMA's: earlier writers do not matter
-            step = int(args2.split()[0], 0) + 1 if op2 == "s_nop" else 1
-            stack.extend((p, ws + step) for p in preds[j])
+            i, ws, regs = stack.pop()
+            _ai, op_i, args_i, t_i = ins[i]
+            step = int(args_i.split()[0], 0) + 1 if op_i == "s_nop" else 1
+            after = ws + (step if i != j or ws else 0)
+            nexts = []
+            if i + 1 < len(ins) and op_i not in _END_FLOW:
+                nexts.append(i + 1)
+            if t_i is not None and (op_i.startswith("s_cbranch") or op_i == "s_branch") and t_i in index:
+                nexts.append(index[t_i])
+            for k in nexts:
+                if after >= MFMA_WAIT[op] or (k, after, regs) in seen:
+                    continue
+                seen.add((k, after, regs))
+                a_k, op_k, args_k, _tk = ins[k]
+                left = regs
+                if op_k.startswith("v_"):
+                    dest, srcs = _operands(args_k)
+                    if op_k.startswith("v_mfma"):
+                        left = regs - dest
+                    elif regs & (dest | srcs):
+                        found.append((hex(a_k), op_k, args_k, after))
+                        continue
+                if left:
+                    stack.append((k, after, left))
     return found
 
 
-def test_mfma_results_wait_on_every_path(device_asm):
-    fns = _functions(device_asm)
+@pytest.fixture(scope="module")
+def device_functions(device_asm):
+    return _functions(device_asm)
+
+
+def test_mfma_results_wait_on_every_path(device_functions):
+    fns = device_functions
     used = {op for ins in fns.values() for _a, op, _x, _t in ins if op.startswith("v_mfma")}
     assert used == set(MFMA_WAIT)
     bad = {name: h[:3] for name, ins in fns.items() if (h := _mfma_hazards(ins))}
@@ -144,14 +151,14 @@ def test_the_wait_check_tells_the_shapes_apart(op, short):
 
 
 # ---------------------------------------------------------------- M0 and LDS DMA
-def test_m0_is_only_set_for_lds_dma(device_asm):
+def test_m0_is_only_set_for_lds_dma(device_functions):
     """The tokenwise ring kernel issues its LDS-DMA loads from inline asm
     that sets M0 (the LDS base of the load) itself. The compiler reserves M0
     and does not expect the asm to change it, so the shipped code must use
     M0 nowhere else: every reference to m0 is that s_mov, followed by the
     one wait state and the load, and every LDS-DMA load has its own M0 set
     right before it."""
-    fns = _functions(device_asm)
+    fns = device_functions
     loads = 0
     for name, ins in fns.items():
         for k, (_a, op, args, _t) in enumerate(ins):
