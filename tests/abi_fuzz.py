@@ -40,6 +40,8 @@ SIGNATURES = {
     "actune_tokenwise_linear": [P, I, P, P, I, P, P, I, P, I, L, L, L, I, P, L, P],
     "actune_tokenwise_linear_x": [P, I, P, P, I, P, P, I, P, I, L, L, L, I, P, L, P],
     "actune_tokenwise_linear_multi": [P, I, P, I, P, I, ctypes.POINTER(TwTarget), I, I, I, L, L, L, I, P, L, P],
+    "actune_weight_candidates": [P, I, P, I, L, L, I, I, P, P, P],
+    "actune_candidate_select": [P, P, P, I, L, L, P, P, P, P],
 }
 
 MS = [-1, 0, 1, 2, 8, 17, 64, 65, 512, 1024, 1025, 2**31, 2**40]
@@ -48,6 +50,7 @@ KS = [-64, 0, 1, 64, 100, 128, 4096, 11008, 65536, 2**31, 2**40]
 WIDTHS = [-1, 0, 1, 2, 3, 4, 8, 16]
 CODES = [-2, -1, 0, 1, 2, 3, 5, 6, 99]
 CONFIGS = [-2, -1, 0, 3, 9, 10, 14, 16, 17]
+COUNTS = [-1, 0, 1, 9, 65535, 65536, 2**31 - 1]  # candidates
 
 
 def main(path, calls):
@@ -95,6 +98,13 @@ def main(path, calls):
         status("tokenwise_linear_multi", lib.actune_tokenwise_linear_multi(
             None, lay2, None, dt, None, lay, tw_targets if nt >= 0 else None, nt, dt, dt2, m, n, k, cfg, None,
             ws, None), m)
+        r = rng.choice(COUNTS)  # without candidates the calls are empty
+        status("weight_candidates", lib.actune_weight_candidates(None, dt, None, r, n, k, w, a, None, None, None), r)
+        status("candidate_select", lib.actune_candidate_select(None, None, None, r, m, n, None, None, None, None), r)
+        # misaligned buffers are named before anything is launched
+        odd = ctypes.c_void_p(0x1001)
+        status("weight_candidates", lib.actune_weight_candidates(odd, 0, odd, 1, 16, 64, 4, 8, odd, odd, None), 1)
+        status("candidate_select", lib.actune_candidate_select(odd, odd, odd, 1, 4, 16, odd, odd, odd, None), 1)
     for b in bad[:20]:
         print("bad", b)
     print(f"{calls} rounds, {len(bad)} bad")

@@ -10,6 +10,7 @@
 // config selection and launch geometry, then fail at the launch on a machine
 // without a GPU (ACTUNE_ERR_DEVICE). Run it only where no GPU is visible:
 // with a GPU, the second half would launch kernels on host memory.
+#include <climits>
 #include <cstdio>
 #include <cstdint>
 #include <random>
@@ -64,6 +65,12 @@ int main(int argc, char** argv) {
     st("tw_linear", actune_tokenwise_linear(B, lay2, B, B, lay, B, B, dt, B, dt2, m, n, k, cfg, B, wsb, nullptr), m);
     st("tw_linear_x", actune_tokenwise_linear_x(B, dt, B, B, lay, B, B, dt, B, dt2, m, n, k, cfg, B, wsb, nullptr), m);
     st("tw_linear_multi", actune_tokenwise_linear_multi(B, lay2, B, dt, B, lay, nt >= 0 ? tw : B, nt, dt, dt2, m, n, k, cfg, B, wsb, nullptr), m);
+    const int cand = (int[]){-1, 0, 1, 9, 65535, 65536, INT_MAX}[rng() % 7];  // without candidates the calls are empty
+    st("weight_candidates", actune_weight_candidates(B, dt, B, cand, n, k, w, a, B, B, nullptr), cand);
+    st("candidate_select", actune_candidate_select(B, B, B, cand, m, n, B, B, B, nullptr), cand);
+    const AnyPtr odd{static_cast<char*>(blk) + 1};
+    st("misaligned candidates", actune_weight_candidates(odd, 0, odd, 1, 16, 64, 4, 8, odd, odd, nullptr) == 1 ? 1 : -1, 1);
+    st("misaligned select", actune_candidate_select(odd, odd, odd, 1, 4, 16, odd, odd, odd, nullptr) == 1 ? 1 : -1, 1);
   }
   if (actune_layout_selftest()) { printf("selftest failed\n"); ++bad; }
   printf("%d rounds, %d bad, %d calls reached a launch\n", rounds, bad, launched);
