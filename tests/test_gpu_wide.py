@@ -58,3 +58,27 @@ def test_planned_siblings_match_single_calls(W, A, m, ns, k):
             cols = np.sort(np.random.default_rng(n).choice(n, size=24, replace=False))
             want = O.linear(a_codes, scales, codes, wscale, None, bounds=canonical_bounds(k // 64), cols=cols)
             np.testing.assert_array_equal(bits(out)[:, cols], O.round_out(want, "bf16"), err_msg=f"n={n}")
+
+
+# The dots mode of configs 3-6 runs the prefill kernel, so the integer dots of the wide-tile kernel are read from its fp32
+# outputs: with a weight scale of 1 and an activation scale of 1 in one group and 0 in the others an output is that
+# group's dot (at most 2^20: exact). Ragged quads; 17 quads (chunks of one and two quads, sets of a K split out of step).
+@pytest.mark.parametrize("W,A", [(w, a) for w in (2, 4, 8) for a in (2, 4, 8)])
+@pytest.mark.parametrize("m,n,k", [(35, 70, 448), (130, 33, 4352)])
+def test_wide_tile_group_dots_are_exact(W, A, m, n, k):
+    gen = torch.Generator().manual_seed(m + n + k)
+    a_codes = torch.randint(-(1 << (A - 1)), 1 << (A - 1), (m, k), generator=gen, dtype=torch.int8)
+    w_codes = torch.randint(-(1 << (W - 1)), 1 << (W - 1), (n, k), generator=gen, dtype=torch.int8)
+    a_codes[0], w_codes[0] = -(1 << (A - 1)), -(1 << (W - 1))  # the largest dot
+    packed_a = torch.from_numpy(O.pack_rows(a_codes.numpy(), A)).to(DEV)
+    packed_w = torch.from_numpy(O.pack_rows(w_codes.numpy(), W)).to(DEV)
+    ones = torch.ones(n, device=DEV)
+    groups = k // 64
+    for g in range(groups) if groups < 8 else (0, 3, 4, 30, 35, 63, 66, 67):
+        scales = torch.zeros(m, groups, device=DEV)
+        scales[:, g] = 1
+        part = slice(64 * g, 64 * g + 64)
+        want = (a_codes[:, part].double() @ w_codes[:, part].double().T).float()
+        for config in (3, 4, 5, 6):
+            out = _native.grouped_linear(packed_a, scales, packed_w, ones, None, (m, k), W, A, config, out_dtype=torch.float32)
+            assert torch.equal(out.cpu(), want), (config, g)
