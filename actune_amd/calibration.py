@@ -69,17 +69,6 @@ def activation_reference(value, bits, group_size=64):
     return deq.reshape(shape)
 
 
-def _ratios(values, device):
-    return torch.tensor([1.0 if v is None else float(v) for v in values], dtype=torch.float32, device=device)
-
-
-def _codes_on_device(weight, w, a, ratio):
-    """weight_codes (quantizers.py:23-94) with torch's GPU division, by the
-    candidates kernel; ratio is a float in (0, 1] or None."""
-    packed, scale = _native.weight_candidates(weight.detach().contiguous(), _ratios((ratio,), weight.device), w, a)
-    return _unpack_codes(packed, w, weight.shape[1]), scale
-
-
 def _outputs(a_codes, weight, w, a, ratios):
     """fp32 outputs [M, R * N] of the packed GEMM for the codes of x against
     the weight candidates of every ratio, one below the other."""
@@ -87,13 +76,6 @@ def _outputs(a_codes, weight, w, a, ratios):
     packed, scale = _native.weight_candidates(weight, ratios, w, a)
     return _native.grouped_linear(a_packed, a_scales, packed, scale, None, (a_packed.shape[0], weight.shape[1]), w, a,
                                   out_dtype=torch.float32)
-
-
-def _candidate(x_scaled, weight, w, a, ratio):
-    """fp32 output of the packed GEMM for x_scaled (already divided by the
-    channel scale, in the layer dtype) against weight codes (w, a, ratio)."""
-    return _outputs(_native.quantize_groups(x_scaled, a), weight.detach().contiguous(), w, a,
-                    _ratios((ratio,), weight.device))
 
 
 # fp32 outputs and packed weights of the candidates evaluated at a time
@@ -158,7 +140,7 @@ def calibrate_linear(linear, inputs, row_weights=None, *, budget="w4a4", group_s
     grid = tuple(clip_grid)
     if not all(0 < ratio <= 1 for ratio in grid):
         raise ValueError("Clip ratios must lie in (0, 1]")
-    grid = _ratios(grid, x.device)
+    grid = torch.tensor([float(ratio) for ratio in grid], dtype=torch.float32, device=x.device)
     totals, clips = {}, {}
     for w in (2, 4, 8):
         for a in widths:

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from actune_amd import _native
 from actune_amd import calibration as C
 from oracle import calibration_oracle as CO
 from oracle import oracle as O
@@ -27,7 +28,9 @@ def test_activation_reference_is_the_inference_codebook(A):
 def test_device_codebooks_follow_gpu_division(W, A):
     _, w, _ = seeded_inputs(1, 256, 48, seed=W * 10 + A)
     for ratio in (None, 0.9):
-        codes, scale = C._codes_on_device(w.to(DEV), W, A, ratio)
+        ratios = torch.tensor([1.0 if ratio is None else ratio], device=DEV)
+        packed, scale = _native.weight_candidates(w.to(DEV), ratios, W, A)
+        codes = C._unpack_codes(packed, W, 256)
         want_c, want_s = O.weight_codes(w.float().numpy(), W, A, ratio, gpu_division=True)
         np.testing.assert_array_equal(codes.cpu().numpy(), want_c)
         np.testing.assert_array_equal(scale.cpu().numpy(), want_s)
@@ -38,7 +41,7 @@ def test_candidate_outputs_are_the_packed_gemm_in_fp32(W, A):
     """Each candidate evaluation is the inference GEMM with fp32 output,
     bit-exact against the oracle in the library's canonical order."""
     x, w, _ = seeded_inputs(24, 512, 40, seed=W + A)
-    y = C._candidate(x.to(DEV), w.to(DEV), W, A, 0.95)
+    y = C._outputs(_native.quantize_groups(x.to(DEV), A), w.to(DEV), W, A, torch.tensor([0.95], device=DEV))
     codes, scale = O.weight_codes(w.float().numpy(), W, A, 0.95, gpu_division=True)
     _, a_s, a_c = O.quantize_groups(bits(x), A)
     want = O.linear(a_c, a_s, codes, scale, bounds=canonical_bounds(8))
