@@ -779,9 +779,10 @@ class DecodeGraphPlan:
     outputs out, 34 us a run; issued directly, about 9.) Longer rows add the
     quantizer launch and replay a graph of the three between staging buffers;
     those runs are serialised by a lock. ``graph_replays`` counts the runs of
-    either form."""
+    either form. ``check=False`` leaves the argument checks of the first form
+    to its runs, each of which makes them."""
 
-    def __init__(self, value, weights, residuals, scales, biases):
+    def __init__(self, value, weights, residuals, scales, biases, *, check=True):
         if not 1 <= len(weights) <= _native.MAX_TARGETS:
             raise ValueError(f"a decode plan takes 1 to {_native.MAX_TARGETS} projections")
         self.weights, self.residuals = tuple(weights), tuple(residuals)
@@ -791,11 +792,12 @@ class DecodeGraphPlan:
         self.layout = _decode_layout(self.residuals)
         self.device, self.dtype = value.device, value.dtype
         self.quantize_in_gemm = self.k <= _FUSED_MAX_K
-        self.lock = threading.Lock()
         if self.quantize_in_gemm:
             self._held = ()
-            self._direct(value)  # runs every argument check
+            if check:
+                self._direct(value)
             return
+        self.lock = threading.Lock()
         dev = value.device
         self.input = torch.empty((1, self.k), device=dev, dtype=value.dtype)
         self.activation = torch.empty((1, self.k), device=dev, dtype=torch.int8)
@@ -861,20 +863,22 @@ def graph_plan_key(value, weights, residuals, scales, biases):
 
 
 def graph_decode_linear(owner, value, packed, residual, scale, bias):
-    """Decode of one row through the owner's plan for this key, captured on
+    """Decode of one row through the owner's plan for this key, made on
     first use; the owner keeps its most recently used plans
     (decode_w4a8_triton.py:441-455)."""
     plans = owner.__dict__.setdefault("_decode_graph_plans", OrderedDict())
     key = graph_plan_key(value, (packed,), (residual,), (scale,), (bias,))
     plan = plans.get(key)
     if plan is None:
-        plan = DecodeGraphPlan(value, (packed,), (residual,), (scale,), (bias,))
+        plan = DecodeGraphPlan(value, (packed,), (residual,), (scale,), (bias,), check=False)
+        result = plan.run(value)  # (a call that raises leaves no plan)
         plans[key] = plan
         while len(plans) > _PLANS_PER_MODULE:
             plans.popitem(last=False)
     else:
         plans.move_to_end(key)
-    return plan.run(value).reshape(*value.shape[:-1], packed.shape[1])
+        result = plan.run(value)
+    return result.reshape(*value.shape[:-1], packed.shape[1])
 
 
 def decode_workspace_summary(module):

@@ -212,9 +212,10 @@ def test_split_reduce_columns(m, n, k):
 
 
 def test_w4a8_decode_graph_plan_and_counters():
-    """M = 1 bf16: the module replays its DecodeGraphPlan (quantizer + split-K
-    GEMM in one hipGraph); outputs equal the direct path and the oracle, and
-    the decode counters advance as the reference's do."""
+    """M = 1 bf16: the module runs its DecodeGraphPlan (rows of this length:
+    the split-K GEMM that quantizes the row, and its reduce, issued directly);
+    outputs equal the direct path and the oracle, and the decode counters
+    advance as the reference's do."""
     torch.manual_seed(6)
     lin = torch.nn.Linear(4096, 4096, bias=False, dtype=torch.bfloat16, device=DEV)
     mod = T.W4A8TritonLinear(lin)

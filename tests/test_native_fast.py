@@ -159,3 +159,25 @@ def test_the_extension_is_built_again_for_another_torch(monkeypatch, tmp_path):
     assert not B._binding_stale()
     B.BINDING_STAMP.write_text(B._binding_target().replace(torch.__version__, "1.0.0"))
     assert B._binding_stale()
+
+
+@pytest.mark.gpu
+def test_a_first_decode_launches_once(monkeypatch):
+    from actune_amd.kernels import tokenwise as T
+    layer = T.W4A8TritonLinear(torch.nn.Linear(256, 128, device=DEV, dtype=torch.bfloat16))
+    x = torch.randn(1, 256, device=DEV, dtype=torch.bfloat16)
+    launches = []
+
+    class Counting:
+        def __getattr__(self, name):
+            launches.append(name)
+            return getattr(fast, name)
+
+    fast = N.fast()
+    monkeypatch.setattr(N, "_FAST", Counting())
+    first = layer(x)
+    assert launches.count("tokenwise_decode") == 1
+    assert torch.equal(first, layer(x)) and launches.count("tokenwise_decode") == 2
+    with pytest.raises(RuntimeError):
+        T.graph_decode_linear(layer, x, layer.packed_weight, None, layer.weight_scale[16:32], layer.bias)
+    assert T.decode_workspace_summary(layer)["decode_graph_plan_count"] == 1
