@@ -385,8 +385,7 @@ int packed_default(int64_t M, int64_t N, int64_t K, int W, int A) {
   // per CU (each unpacked weight slot feeds twice the tokens; 2-7% faster at
   // N=16384 M=256 and N=4096 M=1024; W8's 128x64 tiles hold too many
   // registers for two waves per SIMD), and the wide-tile kernel for the
-  // largest problems. Calls under ACTUNE_CONFIG_AUTO above 16 tokens go on to
-  // run_planned.
+  // largest problems. Above 16 tokens plan_codes may leave this choice.
   const int64_t t64 = ((N + 63) / 64) * ((M + 63) / 64);
   if (t64 < 512) return kPrefillFirst + 3;
   if (t64 < 1024) return kPrefillFirst + 2;

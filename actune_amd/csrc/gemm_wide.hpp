@@ -439,19 +439,6 @@ __global__ __launch_bounds__(64 * WN * WM * KS, 2) void gemm_wide(const LinearAr
 
 constexpr int kWideLdsMax = 160 * 1024;  // a gfx950 CU's LDS
 
-// Lets kernel KERN take `bytes` of dynamic LDS on the current device; once
-// per (kernel, device), safe to call from several host threads.
-template <auto KERN>
-inline void allow_wide_lds(int bytes) {
-  static std::atomic<uint64_t> done{0};  // bit d: raised on device d
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;
-  if (bit && (done.load(std::memory_order_acquire) & bit)) return;
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  done.fetch_or(bit, std::memory_order_release);
-}
-
 // One launch over the problems of g (grid y) with geometry (WN, WM, TM, KS).
 template <int W, int A, int WN, int WM, int TM, int KS>
 inline void launch_wide_t(const LinearArgs& g, hipStream_t st) {
@@ -462,10 +449,10 @@ inline void launch_wide_t(const LinearArgs& g, hipStream_t st) {
   const int tm = (g.M + S::BM - 1) / S::BM;
   const dim3 grid((unsigned)((n_max + S::BN - 1) / S::BN * tm), (unsigned)g.nprob);
   if ((g.K / kGroup + 3) / 4 <= kChunks) {
-    if constexpr (S::LDS > 64 * 1024) allow_wide_lds<gemm_wide<W, A, WN, WM, TM, KS, true>>(S::LDS);
+    if constexpr (S::LDS > 64 * 1024) allow_dynamic_lds<gemm_wide<W, A, WN, WM, TM, KS, true>>(S::LDS);
     gemm_wide<W, A, WN, WM, TM, KS, true><<<grid, S::NT * KS, S::LDS, st>>>(g, tm);
   } else {
-    if constexpr (S::LDS > 64 * 1024) allow_wide_lds<gemm_wide<W, A, WN, WM, TM, KS, false>>(S::LDS);
+    if constexpr (S::LDS > 64 * 1024) allow_dynamic_lds<gemm_wide<W, A, WN, WM, TM, KS, false>>(S::LDS);
     gemm_wide<W, A, WN, WM, TM, KS, false><<<grid, S::NT * KS, S::LDS, st>>>(g, tm);
   }
 }

@@ -76,18 +76,18 @@ __device__ __forceinline__ Problem select_problem(const LinearArgs& args, int ti
   return pr;
 }
 
-// Lets kernel KERN take up to kStreamLdsMax bytes of dynamic LDS on the
-// current device (above the default per-launch limit). Done once per
-// (kernel, device); safe to call from several host threads.
+// Lets kernel KERN take up to `bytes` of dynamic LDS on the current device
+// (above the default per-launch limit; every call with one KERN passes the
+// same). Done once per (kernel, device); safe to call from several host
+// threads.
 template <auto KERN>
-inline void allow_dynamic_lds() {
+inline void allow_dynamic_lds(int bytes = (int)kStreamLdsMax) {
   static std::atomic<uint64_t> done{0};  // bit d: raised on device d
   int dev = 0;
   (void)hipGetDevice(&dev);
   const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;
   if (bit && (done.load(std::memory_order_acquire) & bit)) return;
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)kStreamLdsMax);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   done.fetch_or(bit, std::memory_order_release);
 }
 
