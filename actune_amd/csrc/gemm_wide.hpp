@@ -29,8 +29,12 @@
 // would per chunk. A set without a chunk in a round (or with a shorter one)
 // multiplies scales of 0, whose products add nothing.
 //
-// Bound by the rescale: one cvt and one fma per output and group beside 64
-// int8 MACs, half of the int8 MFMA issue rate at best. Measured on MI355X with
+// Bound by the vector pipe: the rescale is one cvt and one fma per output and
+// group beside 64 int8 MACs, half of the int8 MFMA issue rate at best. Counters
+// (profiles/gemm_wide_m512_pmc.md): 2 x 11008x4096 W4A8 at M = 512 vector pipe
+// 65% busy, 16 of its 26 instructions per MFMA the rescale, matrix pipe 20%,
+// waves waiting 20% of the time; 4096x4096 W8A8, one workgroup per CU, 48%, 16%
+// and 38%. Measured on MI355X with
 // the 16x16x64 kernel that it replaced, or the prefill kernel, before:
 // quantizer included, W4A8 11008x4096 at M = 2000 246 -> 182 us, W8A8 4096 x
 // 4096 at M = 512 31.7 -> 28.2; GEMM alone, W8A8 22016x4096 at M = 64 83.8 ->
