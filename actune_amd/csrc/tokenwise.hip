@@ -1348,8 +1348,8 @@ int64_t tiles_of(int64_t M, int64_t N, const Geometry& g) {
 // in flight, and a tile of 96, 128 or (W8) 192 rows reads fewer weight bytes
 // and reads LDS less often per product, so that its round takes 1.2, 1.5 and
 // 2.3 times as long as a 64-row round (in the layouts that unpack the weight
-// tile from K-major fields 1.4 and 2), measured over M = 500-2000 on
-// six layouts. The fewest rounds by that weight win: 1500 x 11008 x 4096
+// tile from K-major fields 1.4 and 2, so that 128 rows never save a round
+// there), measured over M = 500-2000 on six layouts. The fewest rounds by that weight win: 1500 x 11008 x 4096
 // W8A8 123 us at 64 rows, 90 at 96, 97 at 128, 83 at 192 (taken); 2000 x 4096
 // x 4096 W8A8 52, 47, 43 (taken), 50; 1500 x 11008 x 4096 W4A4 111, 85
 // (taken), 91.
@@ -1366,10 +1366,10 @@ Geometry pick_geometry(int64_t M, int64_t N, int wl) {
   }
   const bool fields = km && !w8;
   const Geometry sizes[4] = {base, {2, 3, 4, 0, ks, 3}, {2, 4, 4, 0, ks, km ? 4 : 3}, {2, 6, 4, 0, ks, 4}};
-  const int round[4] = {fields ? 10 : 11, fields ? 14 : 13, fields ? 20 : 17, 25};
+  const int round[4] = {fields ? 10 : 11, fields ? 14 : 13, 17, 25};
   int best = 0;
   int64_t least = INT64_MAX;
-  for (int i = 0; i < (w8 ? 4 : 3); ++i) {
+  for (int i = 0; i < (w8 ? 4 : fields ? 2 : 3); ++i) {
     const int64_t t = round[i] * ((tiles_of(M, N, sizes[i]) + 255) / 256);
     if (t < least) least = t, best = i;
   }
@@ -1500,7 +1500,7 @@ void launch_gemm_g(const TwArgs& a, const Geometry& g, hipStream_t st) {
     } else if (g.mt == 3) {
       launch_ring_t<WL, AL, EPI, 2, 3, 4, KM ? 1 : 2, 3>(a, st);
     } else if (g.mt == 4) {
-      launch_ring_t<WL, AL, EPI, 2, 4, 4, KM ? 1 : 2, KM ? 4 : 3>(a, st);
+      if constexpr (!KM || WL == ACTUNE_TW_KMAJOR_W8) launch_ring_t<WL, AL, EPI, 2, 4, 4, KM ? 1 : 2, KM ? 4 : 3>(a, st);
     } else {
       if constexpr (WL == ACTUNE_TW_KMAJOR_W8) launch_ring_t<WL, AL, EPI, 2, 6, 4, 1, 4>(a, st);
     }

@@ -10,10 +10,11 @@ from actune_amd.kernels import tokenwise as T
 LAYERS = [T.W4A8TritonLinear, T.W8A8TritonLinear, T.W2A8TritonLinear, T.W4A4NativeLinear, T.W2A4NativeLinear, T.W8A4NativeLinear]
 
 
-# tiles of 64 x 128: below 257, below 512, then 64, 96 (192 rows for W8), 128 rows, and a last tile of one row and column
+# the rows of the tile at each size, by layout (W8, K-major fields, row-major): below 257 and below 512 tiles of 64 x 128,
+# then 128/64/128, 192/96/96, 128/64/128, 192/96/96, 64/64/64 and 96/96/96; ragged sizes end in a tile of one row or column
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k", [(33, 130, 128), (300, 8193, 256), (1000, 4096, 128), (1000, 4097, 384), (1990, 4092, 256),
-                                   (1153, 3970, 640)])
+                                   (1153, 3970, 640), (512, 11008, 128), (1500, 5504, 128)])
 @pytest.mark.parametrize("layer", LAYERS)
 def test_rows_do_not_depend_on_the_tile(layer, m, n, k):
     torch.manual_seed(m + n)
